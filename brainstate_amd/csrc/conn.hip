@@ -9,11 +9,15 @@
 //   * numpy's legacy bounded integers: draw = word & mask with mask the smallest 2^j - 1 >=
 //     n_post - 1, redrawn while draw > n_post - 1 (no draw at all when n_post == 1);
 //   * random(): (a * 2^26 + b) / 2^53 with a = word >> 5, b = next word >> 6.
-// The twist is sequential across blocks but splits into three dependency stages within one
-// (i < 227 reads only old words; 227 <= i < 454 reads new words < 227; i >= 454 reads new
-// words < 397), so one workgroup runs only the twists (three barriers per block) for a word
-// budget of expected draws + 12 standard deviations, and parallel passes temper, count the
-// accepted draws per block, scan the counts and place every accepted draw.
+// The twist is sequential from block to block, so the stream is cut into S segments of 2^m
+// blocks and the state at the start of each is found by jump-ahead (mt_jump.h): a segment's 624
+// state words are XORs of words that follow another segment's state, picked by the set bits
+// of x^(jump) mod P.  k_mt_jump runs once per level, each quadrupling the segments whose
+// state is known; k_mt_gen then twists all segments at once, tempering, writing the words and
+// counting the accepted draws on the way (a word budget of expected draws + 12 standard
+// deviations); k_mt_place ranks and places every accepted draw.  8e7 draws below 1e6 (135k
+// blocks): one workgroup twisting every block, then passes to temper, count, scan and place,
+// took 42.5 ms; this form 0.51 ms (jumps 117 us, twists 190, placing 147 = 4.5 TB/s).
 //
 // Without replacement (allow_multi_conn=False) the reference uses its JAX generator
 // (init_indices_without_replace, :39-62), which cannot be reproduced without JAX.  Here each
@@ -21,8 +25,10 @@
 // round, attempt), key = seed) and Lemire's unbiased bounded integers, then redraws the later
 // copy of every repeated value until the row is duplicate-free; the row keeps draw order.
 #include <cmath>
+#include <type_traits>
 
 #include "common.h"
+#include "mt_jump.h"
 
 namespace {
 
@@ -44,157 +50,247 @@ __device__ __forceinline__ uint32_t mt_temper(uint32_t y) {
   return y;
 }
 
-// Rank of word i of a 624-word block among the block's accepted words, given per-(chunk,
-// wave) accept counts s_cw[3][4] (words i = 256 * chunk + 64 * wave + lane).
-__device__ __forceinline__ uint32_t block_rank(const uint32_t (*s_cw)[4], int chunk, int wave,
-                                               uint64_t ballot) {
-  uint32_t r = 0;
-  for (int c = 0; c < chunk; ++c) r += s_cw[c][0] + s_cw[c][1] + s_cw[c][2] + s_cw[c][3];
-  for (int w = 0; w < wave; ++w) r += s_cw[chunk][w];
-  return r + (uint32_t)bs_rank_below(ballot);
-}
+struct MtState {
+  uint32_t x[kMtN];
+};
 
-// Sequential part: the twists only.  Writes `blocks` blocks of 624 untempered state words.
-__global__ __launch_bounds__(kGen) void k_mt_twist(uint32_t seed, int64_t blocks,
-                                                   uint32_t* __restrict__ words) {
-  __shared__ uint32_t st[2][kMtN];
-  const int tid = threadIdx.x;
-  if (tid == 0) {  // init_genrand: inherently sequential, once
-    uint32_t x = seed;
-    for (int i = 0; i < kMtN; ++i) {
-      st[0][i] = x;
-      x = 1812433253u * (x ^ (x >> 30)) + (uint32_t)(i + 1);
-    }
-  }
-  __syncthreads();
-  int cur = 0;
-  for (int64_t b = 0; b < blocks; ++b) {
-    const uint32_t* o = st[cur];
-    uint32_t* nw = st[cur ^ 1];
-    uint32_t* dst = words + b * kMtN;
-    if (tid < kMtN - kMtM) {
-      const uint32_t v = o[tid + kMtM] ^ mt_mix(o[tid], o[tid + 1]);
-      nw[tid] = v;
-      dst[tid] = v;
-    }
-    __syncthreads();
-    if (tid < kMtN - kMtM) {
-      const int i = tid + (kMtN - kMtM);  // 227 .. 453
-      const uint32_t v = nw[i - (kMtN - kMtM)] ^ mt_mix(o[i], o[i + 1]);
-      nw[i] = v;
-      dst[i] = v;
-    }
-    __syncthreads();
-    if (tid < kMtN - 2 * (kMtN - kMtM)) {  // 454 .. 623
-      const int i = tid + 2 * (kMtN - kMtM);
-      const uint32_t v = nw[i - (kMtN - kMtM)] ^ mt_mix(o[i], i + 1 < kMtN ? o[i + 1] : nw[0]);
-      nw[i] = v;
-      dst[i] = v;
-    }
-    __syncthreads();
-    cur ^= 1;
-  }
-}
-
-// Parallel: temper every word in place and count each block's accepted draws.
-__global__ __launch_bounds__(kGen) void k_mt_count(uint32_t* __restrict__ words, int64_t blocks,
-                                                   uint32_t rng, uint32_t mask,
-                                                   uint32_t* __restrict__ counts) {
-  __shared__ uint32_t s_c[4];
-  const int tid = threadIdx.x;
-  for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x) {
-    uint32_t c = 0;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const int i = q * kGen + tid;
-      bool ok = false;
-      if (i < kMtN) {
-        const uint32_t w = mt_temper(words[b * kMtN + i]);
-        words[b * kMtN + i] = w;
-        ok = (w & mask) <= rng;
-      }
-      c += (uint32_t)__popcll(bs_ballot(ok));
-    }
-    if (bs_lane() == 0) s_c[tid / BS_WAVE] = c;
-    __syncthreads();
-    if (tid == 0) counts[b] = s_c[0] + s_c[1] + s_c[2] + s_c[3];
-    __syncthreads();
-  }
-}
-
-// One workgroup: ofs[b] = accepted draws before block b (ofs[blocks] = all); info[0] = blocks,
-// info[1] = 0 when nothing is drawn (else k_mt_place records the position), info[2] = all.
-__global__ __launch_bounds__(1024) void k_mt_scan(const uint32_t* __restrict__ counts,
-                                                  int64_t blocks, int64_t need,
-                                                  int64_t* __restrict__ ofs,
+// Segment 0's state; the states that k_mt_jump accumulates into cleared; info[0] = blocks,
+// info[1] = 0 when nothing is drawn (else k_mt_place records the position, -1 until then).
+__global__ __launch_bounds__(kGen) void k_mt_init(MtState s0, int32_t segs, int64_t blocks,
+                                                  int64_t need, uint32_t* __restrict__ states,
                                                   int64_t* __restrict__ info) {
-  __shared__ int64_t part[1024];
-  const int64_t per = (blocks + 1023) / 1024;
-  const int64_t lo = threadIdx.x * per;
-  const int64_t hi = lo + per < blocks ? lo + per : blocks;
-  int64_t c = 0;
-  for (int64_t b = lo; b < hi; ++b) c += counts[b];
-  part[threadIdx.x] = c;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int64_t acc = 0;
-    for (int t = 0; t < 1024; ++t) {
-      const int64_t v = part[t];
-      part[t] = acc;
-      acc += v;
-    }
-    ofs[blocks] = acc;
+  for (int64_t i = (int64_t)blockIdx.x * kGen + threadIdx.x; i < (int64_t)segs * kMtN;
+       i += (int64_t)gridDim.x * kGen)
+    states[i] = i < kMtN ? s0.x[i] : 0u;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     info[0] = blocks;
     info[1] = need == 0 ? 0 : -1;
-    info[2] = acc;
-  }
-  __syncthreads();
-  int64_t acc = part[threadIdx.x];
-  for (int64_t b = lo; b < hi; ++b) {
-    ofs[b] = acc;
-    acc += counts[b];
   }
 }
 
-// Places accepted draws: out[ofs[b] + rank] = off + (word & mask) for ranks below `need`; the
-// draw of rank need - 1 records the stream position after it in info[1].
-__global__ __launch_bounds__(kGen) void k_mt_place(const uint32_t* __restrict__ words,
-                                                   const int64_t* __restrict__ ofs,
-                                                   int64_t blocks, int64_t need, uint32_t rng,
-                                                   uint32_t mask, int32_t off,
-                                                   int32_t* __restrict__ out,
-                                                   int64_t* __restrict__ info) {
-  __shared__ uint32_t s_cw[3][4];
+// Words tid, tid + 227 and tid + 454 of the block that follows `o` (624 words in LDS), for
+// tid < 227 (the third exists for tid < 170).  Word i needs new word i - 227, which the same
+// thread has just formed, so a block needs no exchange but the old words; word 623's mix takes
+// new word 0, which every thread forms for itself (three broadcast reads).
+constexpr int kStep = kMtN - kMtM;          // 227
+constexpr int kThird = kMtN - 2 * kStep;    // 170
+__device__ __forceinline__ void mt_block(const uint32_t* o, int tid, uint32_t (&v)[3]) {
+  const int t = tid < kStep ? tid : 0;
+  const int t3 = tid < kThird ? tid : kThird - 1;
+  const uint32_t a0 = o[t], a1 = o[t + 1], am = o[t + kMtM];
+  const uint32_t b0 = o[t + kStep], b1 = o[t + kStep + 1];
+  const uint32_t c0 = o[t3 + 2 * kStep], cn = o[t3 < kThird - 1 ? t3 + 2 * kStep + 1 : 0];
+  const uint32_t z0 = o[0], z1 = o[1], zm = o[kMtM];
+  const uint32_t c1 = t3 < kThird - 1 ? cn : zm ^ mt_mix(z0, z1);
+  v[0] = am ^ mt_mix(a0, a1);
+  v[1] = v[0] ^ mt_mix(b0, b1);
+  v[2] = v[1] ^ mt_mix(c0, c1);
+}
+
+// Jump polynomials on the device, [e][r - 1] = x^(r * 624 * 2^e) mod P: constants of the
+// generator, uploaded once per device and exponent (jump_table).
+__device__ uint32_t d_jump[mt_jump::kMaxE + 1][3][mt_jump::kWords];
+
+// One level: states of segments [nsrc, 4 nsrc) from those of [0, nsrc); segment r * nsrc + src
+// is `src` advanced by r * nsrc segments, poly[r - 1].  Workgroup = (source, part of the
+// polynomials): it regenerates the source's words x[0, hi) in LDS block by block, then each
+// wave takes a run of 32-bit polynomial words: lane l holds the window of 41 words at i0 + 10 l
+// and XORs the ones the three polynomials' 32 bits (wave-uniform) pick into its 3 x 10
+// outputs, so a window word is read once from LDS for 96 bits instead of once per set bit
+// (one target per workgroup: 69 us for the level from 64 to 256 segments).  The waves meet in
+// LDS, the parts in `states`.  Bound by VALU and branch issue.
+constexpr int kJumpB = 1024;
+constexpr int kJumpW = kJumpB / BS_WAVE;
+constexpr int kJumpT = 10;                       // outputs per lane: 63 lanes cover 624
+constexpr int kJumpR = 3;                        // targets per source
+constexpr int kJumpX = mt_jump::kDeg + kMtN;     // words any set bit can reach
+constexpr int kJumpPad = 640;                    // window words past it are read, never used
+__global__ __launch_bounds__(kJumpB) void k_mt_jump(uint32_t* __restrict__ states, int32_t nsrc,
+                                                    int32_t segs, int32_t parts, int e) {
+  __shared__ __align__(16) uint32_t x[kJumpX + kJumpPad];
+  __shared__ uint32_t s_out[kJumpR][kMtN];
   const int tid = threadIdx.x;
-  const int wave = tid / BS_WAVE;
-  for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x) {
-    const int64_t base = ofs[b];
-    if (base >= need) break;  // ofs is non-decreasing
-    uint32_t w[3];
-    uint64_t bal[3];
-    bool ok[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const int i = c * kGen + tid;
-      ok[c] = false;
-      w[c] = 0;
-      if (i < kMtN) {
-        w[c] = words[b * kMtN + i];
-        ok[c] = (w[c] & mask) <= rng;
+  const int lane = bs_lane();
+  const int wid = __builtin_amdgcn_readfirstlane(tid / BS_WAVE);
+  const int32_t part = blockIdx.x % parts;
+  const int32_t src = (int32_t)(blockIdx.x / parts);
+  const uint32_t* poly = d_jump[e][0];
+  const int32_t per = ((mt_jump::kWords + parts - 1) / parts + kJumpW - 1) / kJumpW;
+  const int32_t w0 = (part * kJumpW + wid) * per;                      // this wave's words
+  const int32_t w1 = w0 + per < mt_jump::kWords ? w0 + per : mt_jump::kWords;
+  const int32_t last = (part + 1) * kJumpW * per * 32 + kMtN;          // words the part reads
+  const int32_t hi = last < kJumpX ? last : kJumpX;
+  for (int i = tid; i < kMtN; i += kJumpB) x[i] = states[(int64_t)src * kMtN + i];
+  for (int i = tid; i < kJumpR * kMtN; i += kJumpB) s_out[0][i] = 0u;
+  for (int i = kMtN + tid; i < kJumpX + kJumpPad; i += kJumpB) x[i] = 0u;
+  __syncthreads();
+  for (int32_t n0 = kMtN; n0 < hi; n0 += kMtN) {   // 33 blocks at most: within x's padding
+    if (tid < kGen) {
+      uint32_t v[3];
+      mt_block(x + n0 - kMtN, tid, v);
+      if (tid < kStep) {
+        x[n0 + tid] = v[0];
+        x[n0 + tid + kStep] = v[1];
       }
-      bal[c] = bs_ballot(ok[c]);
-      if (bs_lane() == 0) s_cw[c][wave] = (uint32_t)__popcll(bal[c]);
+      if (tid < kThird) x[n0 + tid + 2 * kStep] = v[2];
     }
     __syncthreads();
+  }
+  uint32_t acc[kJumpR][kJumpT];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      if (ok[c]) {
-        const int64_t r = base + block_rank(s_cw, c, wave, bal[c]);
-        if (r < need) out[r] = off + (int32_t)(w[c] & mask);
-        if (r == need - 1) info[1] = b * kMtN + c * kGen + tid + 1;
+  for (int q = 0; q < kJumpR; ++q)
+#pragma unroll
+    for (int j = 0; j < kJumpT; ++j) acc[q][j] = 0u;
+  for (int32_t w = w0; w < w1; ++w) {
+    uint32_t bits[kJumpR];
+#pragma unroll
+    for (int q = 0; q < kJumpR; ++q)
+      bits[q] = src + (q + 1) * nsrc < segs
+                    ? __builtin_amdgcn_readfirstlane(poly[q * mt_jump::kWords + w]) : 0u;
+    uint32_t r[31 + kJumpT];
+    const uint32_t* p = x + w * 32 + lane * kJumpT;
+#pragma unroll
+    for (int k = 0; k < 31 + kJumpT; ++k) r[k] = p[k];
+#pragma unroll
+    for (int k = 0; k < 32; ++k) {
+#pragma unroll
+      for (int q = 0; q < kJumpR; ++q) {
+        if ((bits[q] >> k) & 1u) {
+#pragma unroll
+          for (int j = 0; j < kJumpT; ++j) acc[q][j] ^= r[k + j];
+        }
       }
     }
+  }
+#pragma unroll
+  for (int q = 0; q < kJumpR; ++q)
+#pragma unroll
+    for (int j = 0; j < kJumpT; ++j)
+      if (lane * kJumpT + j < kMtN) atomicXor(&s_out[q][lane * kJumpT + j], acc[q][j]);
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kJumpR; ++q) {
+    const int32_t tgt = src + (q + 1) * nsrc;
+    if (tgt >= segs) break;
+    for (int i = tid; i < kMtN; i += kJumpB) {
+      uint32_t* d = states + (int64_t)tgt * kMtN + i;
+      if (parts == 1) *d = s_out[q][i];
+      else atomicXor(d, s_out[q][i]);
+    }
+  }
+}
+
+// Segment s: its 2^m blocks twisted one after another from its state, every word tempered and
+// written; lofs[b] = draws accepted in the segment before block b, segtot[s] = in all of it.
+// Waves 0-3 form block b from the old words while waves 4-7 temper, store and count block
+// b - 1: one barrier per block, and the chain from block to block holds the twist alone (all
+// in the same four waves: 0.36 us per block).
+constexpr int kGenB = 2 * kGen;
+__global__ __launch_bounds__(kGenB) void k_mt_gen(const uint32_t* __restrict__ states, int m,
+                                                  int64_t blocks, uint32_t rng, uint32_t mask,
+                                                  uint32_t* __restrict__ words,
+                                                  uint32_t* __restrict__ lofs,
+                                                  uint32_t* __restrict__ segtot) {
+  __shared__ uint32_t st[2][kMtN];
+  __shared__ uint32_t s_c[2][kGen / BS_WAVE];
+  const bool twist = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kGen) == 0;
+  const int tid = threadIdx.x % kGen;
+  const int64_t b0 = (int64_t)blockIdx.x << m;
+  const int32_t nb = (int32_t)((1LL << m) < blocks - b0 ? (1LL << m) : blocks - b0);
+  for (int i = threadIdx.x; i < kMtN; i += kGenB)
+    st[0][i] = states[(int64_t)blockIdx.x * kMtN + i];
+  __syncthreads();
+  uint32_t run = 0;
+  // iteration b: block b from st[b & 1] into the other half, while st[b & 1] (block b - 1) is
+  // written out; counts of block b - 1 are added up in iteration b + 1
+  const bool third = tid < kMtN - 2 * kGen;
+  const int t2 = third ? tid + 2 * kGen : kMtN - 1;
+  auto step = [&](int32_t b, auto half) {
+    constexpr int h = decltype(half)::value;
+    const uint32_t* o = st[h];
+    uint32_t* nw = st[h ^ 1];
+    if (twist) {
+      if (b < nb) {
+        uint32_t v[3];
+        mt_block(o, tid, v);
+        if (tid < kStep) {
+          nw[tid] = v[0];
+          nw[tid + kStep] = v[1];
+        }
+        if (tid < kThird) nw[tid + 2 * kStep] = v[2];
+      }
+      if (tid == 0 && b >= 2 && b <= nb + 1) {
+        lofs[b0 + b - 2] = run;
+        run += s_c[h ^ 1][0] + s_c[h ^ 1][1] + s_c[h ^ 1][2] + s_c[h ^ 1][3];
+      }
+    } else if (b >= 1 && b <= nb) {
+      const uint32_t x0 = mt_temper(o[tid]), x1 = mt_temper(o[tid + kGen]);
+      const uint32_t x2 = mt_temper(o[t2]);
+      uint32_t* dst = words + (b0 + b - 1) * kMtN;   // wave-uniform base
+      dst[(uint32_t)tid] = x0;
+      dst[(uint32_t)tid + kGen] = x1;
+      if (third) dst[(uint32_t)tid + 2 * kGen] = x2;
+      const uint32_t c = (uint32_t)(__popcll(bs_ballot((x0 & mask) <= rng)) +
+                                    __popcll(bs_ballot((x1 & mask) <= rng)) +
+                                    __popcll(bs_ballot(third && (x2 & mask) <= rng)));
+      if (bs_lane() == 0) s_c[h][tid / BS_WAVE] = c;
+    }
     __syncthreads();
+  };
+  for (int32_t b = 0; b <= nb + 1; b += 2) {
+    step(b, std::integral_constant<int, 0>());
+    step(b + 1, std::integral_constant<int, 1>());
+  }
+  if (threadIdx.x == 0) segtot[blockIdx.x] = run;
+}
+
+// Places accepted draws: out[rank] = word & mask for ranks below `need`; the draw of rank
+// need - 1 records the stream position after it in info[1].  A workgroup takes 2^kPlaceM
+// consecutive blocks of one segment (fewer when segments are shorter), each wave every fourth
+// of them: ten ballots rank a block's words, with no barrier.
+constexpr int kPlaceM = 5;
+__global__ __launch_bounds__(kGen) void k_mt_place(const uint32_t* __restrict__ words,
+                                                   const uint32_t* __restrict__ lofs,
+                                                   const uint32_t* __restrict__ segtot, int m,
+                                                   int64_t blocks, int64_t need, uint32_t rng,
+                                                   uint32_t mask, int32_t* __restrict__ out,
+                                                   int64_t* __restrict__ info) {
+  __shared__ int64_t s_p[kGen / BS_WAVE];
+  const int lane = bs_lane();
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / BS_WAVE));
+  const int pm = m < kPlaceM ? m : kPlaceM;
+  const int64_t bb = (int64_t)blockIdx.x << pm;
+  const int32_t seg = (int32_t)(bb >> m);
+  // accepted draws of the segments before this one
+  int64_t c = 0;
+  for (int32_t s = threadIdx.x; s < seg; s += kGen) c += segtot[s];
+  for (int o = BS_WAVE / 2; o > 0; o >>= 1) c += __shfl_xor(c, o);
+  if (lane == 0) s_p[wid] = c;
+  __syncthreads();
+  const int64_t base0 = s_p[0] + s_p[1] + s_p[2] + s_p[3];
+  for (int k = wid; k < (1 << pm); k += kGen / BS_WAVE) {
+    const int64_t b = bb + k;
+    if (b >= blocks) break;
+    int64_t r = base0 + lofs[b];
+    if (r >= need) break;  // ranks only grow
+    uint32_t w[10];
+#pragma unroll
+    for (int q = 0; q < 10; ++q) {
+      const int i = q * BS_WAVE + lane;
+      w[q] = i < kMtN ? words[b * kMtN + i] : 0xffffffffu;
+    }
+#pragma unroll
+    for (int q = 0; q < 10; ++q) {
+      const int i = q * BS_WAVE + lane;
+      const bool ok = i < kMtN && (w[q] & mask) <= rng;
+      const uint64_t bal = bs_ballot(ok);
+      const int64_t x = r + bs_rank_below(bal);
+      if (ok && x < need) {
+        out[x] = (int32_t)(w[q] & mask);
+        if (x == need - 1) info[1] = b * kMtN + i + 1;
+      }
+      r += __popcll(bal);
+    }
   }
 }
 
@@ -375,23 +471,89 @@ int64_t word_budget(int64_t need, uint32_t rng, int64_t extra) {
   return (int64_t)(mean + 12.0 * sd) + extra + 2 * kMtN;
 }
 
+// Workgroups per source of a level of jumps: levels with few sources split their polynomials
+// (down to 2 or 3 32-bit words per wave) so that the level fills the chip.
+int jump_parts(int64_t srcs) {
+  const int64_t p = 256 / srcs;
+  return (int)(p < 1 ? 1 : (p > 16 ? 16 : p));
+}
+
+// Segments of 2^m blocks.  Few long segments leave the chip idle while they twist, many
+// short ones cost a jump each, and every level of jumps is a launch that regenerates 33 blocks:
+// m minimises the three, with their measured costs (15 us per level, 38 us per target and
+// workgroup, 0.33 / 0.56 / 0.9 us per block with 1 / 2 / 4 segments on a compute unit).  For
+// 135k blocks m = 8 / 9 / 10 took 470 / 455 / 560 us of kernels; short streams stay in one
+// segment (below ~70 blocks) or few (430 blocks, 256k draws: 205 us in one, 91 in 14).
+struct MtPlan {
+  int m, levels;
+  int32_t segs;
+};
+
+MtPlan mt_plan(int64_t blocks) {
+  constexpr double kLevelUs = 15.0, kJumpUs = 38.0;
+  constexpr int64_t kMaxSegs = 1024, kCus = 256;
+  MtPlan best{0, 0, 0};
+  double cost = 0.0;
+  for (int m = 0; m <= 22; ++m) {
+    const int64_t segs = (blocks + (1LL << m) - 1) >> m;
+    if (segs > kMaxSegs) continue;
+    int levels = 0;
+    double c = (double)(segs > 1 ? 1LL << m : blocks) *
+               (0.12 + 0.2 * (double)((segs + kCus - 1) / kCus));
+    for (int64_t nsrc = 1; nsrc < segs; nsrc *= 4, ++levels) {
+      const int64_t srcs = segs - nsrc < nsrc ? segs - nsrc : nsrc;
+      const int64_t tgts = (segs < 4 * nsrc ? segs : 4 * nsrc) - nsrc;
+      c += kLevelUs + kJumpUs / jump_parts(srcs) * (double)((tgts + srcs - 1) / srcs);
+    }
+    if (best.segs == 0 || c < cost) {
+      best = MtPlan{m, levels, (int32_t)segs};
+      cost = c;
+    }
+    if (segs == 1) break;
+  }
+  return best;
+}
+
+// Makes d_jump[e] valid on the current device: a synchronous copy the first time, so every
+// stream sees it from then on.
+int jump_table(int e) {
+  constexpr int kDevs = 64;
+  static std::mutex mu;
+  static bool done[kDevs][mt_jump::kMaxE + 1];
+  int dev = 0;
+  BS_CHECK_HIP(hipGetDevice(&dev));
+  BS_CHECK_ARG(e >= 0 && e <= mt_jump::kMaxE && dev < kDevs, "bs_conn_fixed_num: jump 2^%d on "
+               "device %d out of range", e, dev);
+  std::lock_guard<std::mutex> lock(mu);
+  if (done[dev][e]) return BS_OK;
+  constexpr size_t kBytes = 3 * sizeof(mt_jump::Poly);
+  BS_CHECK_HIP(hipMemcpyToSymbol(HIP_SYMBOL(d_jump), mt_jump::powers(e), kBytes, kBytes * e,
+                                 hipMemcpyHostToDevice));
+  done[dev][e] = true;
+  return BS_OK;
+}
+
 struct MtWs {
   int64_t blocks;
-  size_t off_words, off_counts, off_ofs, off_info, bytes;
+  MtPlan plan;
+  size_t off_words, off_lofs, off_tot, off_states, off_info, bytes;
 };
 
 MtWs mt_ws(int64_t need, uint32_t rng, int64_t extra) {
   MtWs w;
   w.blocks = (word_budget(need, rng, extra) + kMtN - 1) / kMtN;
+  w.plan = mt_plan(w.blocks);
   size_t o = 0;
-  w.off_words = o;
-  o += ((size_t)w.blocks * kMtN * 4 + 255) & ~(size_t)255;
-  w.off_counts = o;
-  o += ((size_t)w.blocks * 4 + 255) & ~(size_t)255;
-  w.off_ofs = o;
-  o += ((size_t)(w.blocks + 1) * 8 + 255) & ~(size_t)255;
-  w.off_info = o;
-  o += 256;
+  auto take = [&](size_t bytes) {
+    const size_t at = o;
+    o += (bytes + 255) & ~(size_t)255;
+    return at;
+  };
+  w.off_words = take((size_t)w.blocks * kMtN * 4);
+  w.off_lofs = take((size_t)w.blocks * 4);
+  w.off_tot = take((size_t)w.plan.segs * 4);
+  w.off_states = take((size_t)w.plan.segs * kMtN * 4);
+  w.off_info = take(256);
   w.bytes = o;
   return w;
 }
@@ -429,22 +591,38 @@ extern "C" int bs_conn_fixed_num(uint32_t seed, int32_t n_pre, int32_t k, int32_
   hipStream_t s = bs_stream(stream);
   char* ws = (char*)workspace;
   uint32_t* words = (uint32_t*)(ws + w.off_words);
-  uint32_t* counts = (uint32_t*)(ws + w.off_counts);
-  int64_t* ofs = (int64_t*)(ws + w.off_ofs);
+  uint32_t* lofs = (uint32_t*)(ws + w.off_lofs);
+  uint32_t* segtot = (uint32_t*)(ws + w.off_tot);
+  uint32_t* states = (uint32_t*)(ws + w.off_states);
   int64_t* info = (int64_t*)(ws + w.off_info);
-  int grid = bs_num_cus() * 8;
-  if ((int64_t)grid > w.blocks) grid = (int)w.blocks;
-  k_mt_twist<<<1, kGen, 0, s>>>(seed, w.blocks, words);
+  const MtPlan& pl = w.plan;
+  BS_CHECK_ARG(pl.segs > 0, "bs_conn_fixed_num: %lld blocks exceed the generator's reach",
+               (long long)w.blocks);
+  MtState s0;
+  mt_jump::seed_state(seed, s0.x);
+  k_mt_init<<<pl.segs < 256 ? pl.segs : 256, kGen, 0, s>>>(s0, pl.segs, w.blocks, need, states,
+                                                           info);
   BS_CHECK_LAUNCH();
-  k_mt_count<<<grid, kGen, 0, s>>>(words, w.blocks, rng, mask, counts);
-  BS_CHECK_LAUNCH();
-  k_mt_scan<<<1, 1024, 0, s>>>(counts, w.blocks, need, ofs, info);
+  for (int d = 0; d < pl.levels; ++d) {
+    const int32_t nsrc = 1 << (2 * d);
+    const int32_t srcs = pl.segs - nsrc < nsrc ? pl.segs - nsrc : nsrc;
+    const int parts = jump_parts(srcs);
+    const int rc = jump_table(pl.m + 2 * d);
+    if (rc) return rc;
+    k_mt_jump<<<srcs * parts, kJumpB, 0, s>>>(states, nsrc, pl.segs, parts, pl.m + 2 * d);
+    BS_CHECK_LAUNCH();
+  }
+  k_mt_gen<<<pl.segs, kGenB, 0, s>>>(states, pl.m, w.blocks, rng, mask, words, lofs, segtot);
   BS_CHECK_LAUNCH();
   if (total > 0) {
     if (need == 0) {  // one target: every index is 0
       k_fill_i32<<<bs_num_cus() * 4, 256, 0, s>>>(indices, total, 0);
     } else {
-      k_mt_place<<<grid, kGen, 0, s>>>(words, ofs, w.blocks, need, rng, mask, 0, indices, info);
+      const int pm = pl.m < kPlaceM ? pl.m : kPlaceM;
+      const int64_t g = (w.blocks + (1LL << pm) - 1) >> pm;
+      BS_CHECK_ARG(g <= INT32_MAX, "bs_conn_fixed_num: too many draws");
+      k_mt_place<<<(int)g, kGen, 0, s>>>(words, lofs, segtot, pl.m, w.blocks, need, rng, mask,
+                                         indices, info);
     }
     BS_CHECK_LAUNCH();
   }
@@ -453,7 +631,7 @@ extern "C" int bs_conn_fixed_num(uint32_t seed, int32_t n_pre, int32_t k, int32_
         words, info, w.blocks * kMtN, n_pre, afferent_ratio, selected);
     BS_CHECK_LAUNCH();
   }
-  int64_t hinfo[3];
+  int64_t hinfo[2];
   BS_CHECK_HIP(hipMemcpyAsync(hinfo, info, sizeof(hinfo), hipMemcpyDeviceToHost, s));
   BS_CHECK_HIP(hipStreamSynchronize(s));
   if (hinfo[1] < 0 || hinfo[1] + extra > w.blocks * kMtN) {

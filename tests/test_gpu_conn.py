@@ -42,6 +42,20 @@ def test_indices_equal_numpy_randint(bs, seed, n_pre, k, n_post):
     assert np.array_equal(idx.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize('need', [1, 30_000, 45_001, 250_000, 1_300_003, 20_000_000])
+@pytest.mark.parametrize('n_post', [1024, 1025, 700_001])
+def test_segmented_stream_equals_numpy(bs, need, n_post):
+    """Streams of one segment, of a few, of a last segment cut short, and of every level of
+    jumps, at acceptance 1, 1/2 and 2/3, with the selection that continues the stream."""
+    say('conn segments', need, n_post)
+    r = np.random.RandomState(need % 1000)
+    want = r.randint(0, n_post, size=(need, 1)).astype(np.int32)
+    want_sel = r.random(need) < 0.5
+    idx, sel = bs.ops.conn_fixed_num(need % 1000, need, 1, n_post, 0.5)
+    assert np.array_equal(idx.cpu().numpy(), want)
+    assert np.array_equal(sel.cpu().numpy(), want_sel)
+
+
 @pytest.mark.parametrize('seed,n_pre,k,n_post,ratio', [(3, 500, 20, 800, 0.5),
                                                        (4, 1000, 7, 1, 0.3),
                                                        (6, 333, 0, 10, 0.9),
