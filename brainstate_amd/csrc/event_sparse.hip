@@ -273,13 +273,28 @@ __global__ __launch_bounds__(kBlock) void k_matvec(const T* __restrict__ spk, in
   }
 }
 
+// gw[0] += the sum over the workgroup's waves of their (wave-uniform) v: one atomic per
+// workgroup.  Called by every wave that has not ended.  (One per active row made the shared
+// weight's gradient of 100k rows of 128 synapses take 1.27 ms.)
+template <int kWaves>
+__device__ __forceinline__ void block_atomic_sum(float v, float* gw) {
+  __shared__ float s_v[kWaves];
+  const int wid = threadIdx.x / BS_WAVE;
+  if (bs_lane() == 0) s_v[wid] = v;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  float t = s_v[0];
+  for (int u = 1; u < kWaves; ++u) t += s_v[u];
+  if (t != 0.0f) bs_atomic_add_f32(gw, t);
+}
+
 constexpr int kVjpU = 8;  // 64-synapse chunks per wave and round in k_matvec_vjp
 
 // Reverse mode of the event mat-vec y[j] = sum_{i,k: idx[i,k]=j} x[i] * w[i,k] (x = spike
 // value; 1 for byte spikes): one wave per pre row i gathers g[idx[i,k]] over the row and
 //   grad_x[i]   = sum_k w[i,k] * g[idx[i,k]]            (lane partials, then a wave sum)
 //   grad_w[i,k] = x[i] * g[idx[i,k]]                    (per-synapse weights)
-//   grad_w[0]  += x[i] * sum_k g[idx[i,k]]              (homogeneous weight; one atomic/row)
+//   grad_w[0]  += x[i] * sum_k g[idx[i,k]]              (homogeneous weight)
 // Synapses with out-of-range targets contribute nothing, as in the forward pass.
 template <typename T, bool kCsr, bool kHet>
 __global__ __launch_bounds__(kBlock) void k_matvec_vjp(const T* __restrict__ spk, int32_t n_pre,
@@ -293,6 +308,7 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp(const T* __restrict__ spk
   const int lane = bs_lane();
   const int64_t nw = (int64_t)gridDim.x * (kBlock / BS_WAVE);
   const int32_t nnz = kCsr ? indptr[n_pre] : 0;
+  float sw = 0.0f;
   for (int64_t row = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / BS_WAVE; row < n_pre;
        row += nw) {
     int64_t beg, end;
@@ -337,11 +353,220 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp(const T* __restrict__ spk
       sx += __shfl_xor(sx, o);
       sg += __shfl_xor(sg, o);
     }
-    if (lane == 0) {
-      if (gx) gx[row] = sx;
-      if (!kHet && gw && xv != 0.0f) bs_atomic_add_f32(gw, xv * sg);
+    if (lane == 0 && gx) gx[row] = sx;
+    if (!kHet && xv != 0.0f) sw += xv * sg;
+  }
+  if (!kHet && gw) block_atomic_sum<kBlock / BS_WAVE>(sw, gw);
+}
+
+// Sum over the wave in k_matvec_vjp's order (lane l with l ^ 32, then 16, 8, 4, 2, 1): after the
+// exchange at distance 8 the values repeat every 8 lanes, so a rotation by 4 inside 16 lanes
+// meets the same value as the exchange at distance 4.
+__device__ __forceinline__ float wave_sum_xor(float v) {
+  v += __shfl_xor(v, 32);
+  v += __shfl_xor(v, 16);
+#define BS_DPP(x, ctrl) \
+  __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xF, 0xF, true))
+  v += BS_DPP(v, 0x128);  // row_ror:8
+  v += BS_DPP(v, 0x124);  // row_ror:4
+  v += BS_DPP(v, 0x4E);   // quad_perm [2, 3, 0, 1]
+  v += BS_DPP(v, 0xB1);   // quad_perm [1, 0, 3, 2]
+#undef BS_DPP
+  return v;
+}
+
+// The same gradients (fixed fan-out) with g read from LDS.  A gather of g from L2 moves a whole
+// 128-byte line for 4 bytes, which holds k_matvec_vjp at ~2e11 gathers/s, fewer when the
+// synapses come from HBM.  Here one workgroup per compute unit streams the synapses of its
+// rows while ranges of kLvR posts of g pass through two LDS buffers: 4 waves load the next
+// range into one buffer while 12 waves pick the values of their targets out of the other, with
+// one barrier per range.  Each of the 12 waves holds kLvS chunks of 64 synapses at a time --
+// kLvS / CP rows of CP chunks, or 16 chunks of a longer row -- with the next pass's indices
+// and this pass's weights in flight.  An index outside the range reads the zero slot behind
+// it; at most one range holds a target, so OR-ing the bits of all ranges is exact.  Up to two
+// ranges stay in LDS for the whole launch.
+// Loads and stores of a pass are unconditional (lanes past the row's end repeat its last
+// synapse, rows past the wave's last repeat that row, with the same values), so that the wait
+// for the next indices counts only what was issued after them.
+// Every row is summed as k_matvec_vjp sums it, bit for bit.
+constexpr int kLvB = 1024;
+constexpr int kLvR = 20416;                       // posts per range (two ranges fill LDS)
+template <typename T, int CP, bool kHet, bool kGw, bool kMulti>
+__global__ __launch_bounds__(kLvB) void k_matvec_vjp_lds(
+    const T* __restrict__ spk, int32_t n_pre, const int32_t* __restrict__ indices, int32_t k,
+    const float* __restrict__ w, float w_homo, int32_t n_post, const float* __restrict__ g,
+    float* __restrict__ gx, float* __restrict__ gw) {
+  constexpr int kLvS = kMulti ? 32 : 16;              // chunks per wave and pass
+  constexpr int kLvW = kMulti ? 12 : 16;              // waves that own rows
+  constexpr int kLvF = kMulti ? 256 : kLvB;           // threads that fill LDS (the last ones)
+  constexpr int kR = kLvS / CP;                       // rows per pass
+  __shared__ __align__(16) uint32_t s_g[2][kLvR + 16];  // [kLvR]: the zero slot
+  const int lane = bs_lane();
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / BS_WAVE));
+  const int64_t nw = (int64_t)gridDim.x * kLvW;
+  const int32_t nblk = (k + CP * BS_WAVE - 1) / (CP * BS_WAVE);  // > 1 only for CP = 16
+  // the same number of passes in every wave: the ranges change at barriers
+  const int32_t passes = (int32_t)(((n_pre + nw - 1) / nw + kR - 1) / kR) * nblk;
+  const int32_t nr = (n_post + kLvR - 1) / kLvR;      // at most 2 unless kMulti
+  // range q by kLvF threads: into registers (16-byte loads, all in flight), then to s_g[buf]
+  constexpr int kU = (kLvR / 4 + kLvF - 1) / kLvF;
+  static_assert(4 * kU * kLvF >= kLvR + 4, "the zero slot is written with its range");
+  const bool al = ((uintptr_t)g & 15) == 0;
+  auto length = [&](int32_t q) { return n_post - q * kLvR < kLvR ? n_post - q * kLvR : kLvR; };
+  auto load = [&](int32_t q, int tid, uint4 (&v)[kU], uint32_t (&tail)[3]) {
+    const int32_t len = length(q), len4 = len & ~3;
+    const uint32_t* p = (const uint32_t*)g + (int64_t)q * kLvR;
+    if (!al || len4 == 0) return;                     // store() reads g itself
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int i = 4 * (tid + u * kLvF);
+      v[u] = *(const uint4*)(p + (i < len4 ? i : len4 - 4));
+    }
+#pragma unroll
+    for (int e = 0; e < 3; ++e) tail[e] = p[len4 + e < len ? len4 + e : len - 1];
+  };
+  auto store = [&](int32_t q, int buf, int tid, const uint4 (&v)[kU], const uint32_t (&tail)[3]) {
+    const int32_t len = length(q), len4 = len & ~3;
+    if (!al || len4 == 0) {
+      const uint32_t* p = (const uint32_t*)g + (int64_t)q * kLvR;
+      for (int i = tid; i < kLvR + 16; i += kLvF) s_g[buf][i] = i < len ? p[i] : 0u;
+      return;
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int i = 4 * (tid + u * kLvF);
+      const bool full = i < len4, cut = i == len4;
+      uint4 x;
+      x.x = full ? v[u].x : (cut && len4 < len ? tail[0] : 0u);
+      x.y = full ? v[u].y : (cut && len4 + 1 < len ? tail[1] : 0u);
+      x.z = full ? v[u].z : (cut && len4 + 2 < len ? tail[2] : 0u);
+      x.w = full ? v[u].w : 0u;
+      if (i < kLvR + 16) *(uint4*)(s_g[buf] + i) = x;
+    }
+  };
+  // compute units of one XCD start at different ranges, so that they do not all read the same
+  // lines of g at once
+  const int32_t q0 = kMulti ? (int32_t)((blockIdx.x / 8) % nr) : 0;
+  if (kLvF == kLvB || wid >= kLvW) {  // the filling waves
+    const int tid = (int)threadIdx.x - (kLvB - kLvF);
+    uint4 v[kU];
+    uint32_t tail[3];
+    int32_t q = q0;
+    load(q, tid, v, tail);
+    store(q, 0, tid, v, tail);
+    if constexpr (!kMulti) {
+      if (nr == 2) {
+        load(1, tid, v, tail);
+        store(1, 1, tid, v, tail);
+      }
+    } else {
+      // step t reads range q0 + t (mod nr) from s_g[t & 1]; the next one is stored meanwhile,
+      // and the one after it is on its way across the barrier
+      const int64_t steps = (int64_t)passes * nr;
+      auto ahead = [&](int64_t t) {
+        q = q + 1 == nr ? 0 : q + 1;
+        if (t < steps) load(q, tid, v, tail);
+      };
+      ahead(1);
+      __syncthreads();
+      for (int64_t t = 0; t < steps; ++t) {
+        if (t + 1 < steps) store(q, (int)((t + 1) & 1), tid, v, tail);
+        ahead(t + 2);
+        __syncthreads();
+      }
+      if (!kHet && gw) block_atomic_sum<kLvB / BS_WAVE>(0.0f, gw);
+      return;
     }
   }
+  __syncthreads();
+  const int64_t wv = (int64_t)blockIdx.x * kLvW + wid;
+  const int64_t r0 = n_pre * wv / nw;                 // this wave's rows [r0, r0 + rows)
+  const int32_t rows = (int32_t)(n_pre * (wv + 1) / nw - r0);
+  const int32_t lastr = rows > 0 ? rows - 1 : 0;      // repeated past the end (r0 < n_pre)
+  auto rowat = [&](int32_t r) -> int64_t { return (r0 + (r < lastr ? r : lastr)) * k; };
+  // byte offset in its row of this lane's synapse in chunk c of a block that starts at kb
+  auto syn = [&](int32_t kb, int c, int ln) -> uint32_t {
+    const int32_t t = kb + c * BS_WAVE + ln;
+    return (uint32_t)(t < k ? t : k - 1) * 4u;
+  };
+  // the lane number, hidden from the compiler: it would keep the offsets of one walk over the
+  // chunks for the next and spill
+  auto hidden = [&]() {
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    return ln;
+  };
+  auto rd = [](const void* p, uint32_t off) { return *(const uint32_t*)((const char*)p + off); };
+  uint32_t jj[kLvS];
+  auto load_idx = [&](int32_t r, int32_t b) {
+    const int ln = hidden();
+#pragma unroll
+    for (int s = 0; s < kLvS; ++s) jj[s] = rd(indices + rowat(r + s / CP), syn(b, s % CP, ln));
+  };
+  load_idx(0, 0);
+  float cx[kR], cg[kR], sw = 0.0f;                    // lane sums carried over a row's blocks
+  int32_t row = 0, kb = 0;                            // this pass: rows row .. row + kR - 1
+  int step = 0;
+  for (int32_t pass = 0; pass < passes; ++pass) {
+    uint32_t gj[kLvS];
+    float wt[kLvS];
+    // lane r: the spike value of row r of the pass
+    const float xl = (float)spk[r0 + (row + lane < lastr ? row + lane : lastr)];
+#pragma unroll
+    for (int s = 0; s < kLvS; ++s) {
+      jj[s] = (jj[s] < (1u << 29) ? jj[s] : 1u << 29) * 4u;   // byte offset in g
+      gj[s] = 0u;
+    }
+    for (int32_t qq = 0, q = q0; qq < nr; ++qq, q = q + 1 == nr ? 0 : q + 1) {
+      const uint32_t lo = (uint32_t)q * kLvR * 4u;
+      const char* sgp = (const char*)s_g[kMulti ? step & 1 : q];
+      if (qq + 1 == nr) {                             // weights: in flight during the last range
+        const int ln = hidden();
+#pragma unroll
+        for (int s = 0; s < kLvS; ++s)
+          wt[s] = kHet ? __uint_as_float(rd(w + rowat(row + s / CP), syn(kb, s % CP, ln)))
+                       : w_homo;
+      }
+#pragma unroll
+      for (int s = 0; s < kLvS; ++s) {
+        const uint32_t u = jj[s] - lo;
+        gj[s] |= *(const uint32_t*)(sgp + (u < kLvR * 4u ? u : kLvR * 4u));
+      }
+      ++step;
+      if (kMulti) __syncthreads();
+    }
+    // the next pass's indices (past the end: the last row's again), in flight from here
+    const bool wrap = CP < 16 || kb + CP * BS_WAVE >= k;
+    const int32_t nrow = wrap ? row + kR : row, nkb = wrap ? 0 : kb + CP * BS_WAVE;
+    load_idx(nrow, nkb);
+    const int ln = hidden();
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+      const float xv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(xl), r));
+      float sx = kb ? cx[r] : 0.0f, sg = kb ? cg[r] : 0.0f;
+#pragma unroll
+      for (int c = 0; c < CP; ++c) {
+        const float gv = __uint_as_float(gj[r * CP + c]);
+        const bool in = kb + c * BS_WAVE + ln < k;
+        if (kGw) *(float*)((char*)(gw + rowat(row + r)) + syn(kb, c, ln)) = xv * gv;
+        sx += in ? wt[r * CP + c] * gv : 0.0f;
+        if (!kHet) sg += in ? gv : 0.0f;
+      }
+      if (CP == 16) {
+        cx[r] = sx;
+        cg[r] = sg;
+      }
+      if (wrap) {
+        const bool own = row + r < rows;
+        const float vx = wave_sum_xor(sx);
+        if (gx && own && lane == 0) gx[r0 + row + r] = vx;
+        if (!kHet && own && xv != 0.0f) sw += xv * wave_sum_xor(sg);
+      }
+    }
+    row = nrow;
+    kb = nkb;
+  }
+  if (!kHet && gw) block_atomic_sum<kLvB / BS_WAVE>(sw, gw);
 }
 
 // The same gradients for B batch rows in one launch (spk [B, n_pre], g [B, n_post]): one wave
@@ -640,6 +865,29 @@ extern "C" int bs_event_matvec_vjp_batch_f32(const void* spk, int32_t spk_dtype,
   return BS_OK;
 }
 
+namespace {
+
+// Whether k_matvec_vjp_lds is the faster of the two (kernel times, us; L2 gathers / LDS).
+// With g resident (n_post <= 40,832) filling LDS costs ~9 us, the L2 kernel 5 us per 1e6
+// synapses: 10k x 100 synapses 8.7 / 10.7, 2k x 1000 9.2 / 7.9, 20k x 200 19.1 / 12.3,
+// 100k x 200 91 / 43.  With nr > 2 ranges a synapse slot (rows are padded to CP chunks) costs
+// (2.0 + 0.28 nr) 1e-6 us, an L2 gather 4.9e-6, or 7e-6 when the synapses do not stay in the
+// 256 MB memory-side cache: 100k posts, K = 100 (28 % padding) 51 / 54, K = 128 62 / 57,
+// 5k x 1000 28 / 21, 100k x 1000 699 / 318; 400k posts (20 ranges) 359 / 456.
+bool vjp_lds(int32_t n_pre, int32_t k, int32_t n_post, int bytes_per_syn) {
+  const double syn = (double)n_pre * k;
+  if (k >= (1 << 28)) return false;                   // 32-bit byte offsets inside a row
+  const int32_t nr = (int32_t)(((int64_t)n_post + kLvR - 1) / kLvR);
+  if (nr <= 2) return syn >= 1.5e6;
+  if (syn < 3e6) return false;
+  const int64_t cpr = ((int64_t)k + BS_WAVE - 1) / BS_WAVE;
+  const int64_t slots = cpr <= 2 ? cpr : cpr <= 4 ? 4 : cpr <= 8 ? 8 : (cpr + 15) / 16 * 16;
+  const double gather = syn * bytes_per_syn > 256e6 ? 7.0 : 4.9;
+  return (2.0 + 0.28 * nr) * 1.15 * (double)(slots * BS_WAVE) < gather * k;
+}
+
+}  // namespace
+
 extern "C" int bs_event_matvec_vjp_f32(const void* spk, int32_t spk_dtype, int32_t n_pre,
                                        const int32_t* indptr, const int32_t* indices, int32_t k,
                                        const float* w, float w_homo, int32_t n_post,
@@ -664,6 +912,37 @@ extern "C" int bs_event_matvec_vjp_f32(const void* spk, int32_t spk_dtype, int32
       int rc = bs_fill_f32(grad_spk, n_pre, 0.0f, s);
       if (rc) return rc;
     }
+    return BS_OK;
+  }
+  if (!csr && vjp_lds(n_pre, k, n_post, het ? (grad_w ? 12 : 8) : 4)) {
+    const int cpr = (k + BS_WAVE - 1) / BS_WAVE;
+    const int gl = bs_num_cus();
+#define BS_VJPL(T, CP, H, G)                                                               \
+  do {                                                                                     \
+    if (n_post > 2 * kLvR)                                                                 \
+      k_matvec_vjp_lds<T, CP, H, G, true><<<gl, kLvB, 0, s>>>(                             \
+          (const T*)spk, n_pre, indices, k, w, w_homo, n_post, grad_out, grad_spk, grad_w);  \
+    else                                                                                   \
+      k_matvec_vjp_lds<T, CP, H, G, false><<<gl, kLvB, 0, s>>>(                            \
+          (const T*)spk, n_pre, indices, k, w, w_homo, n_post, grad_out, grad_spk, grad_w);  \
+  } while (0)
+#define BS_VJPL2(T, CP)                                                 \
+  do {                                                                  \
+    if (!het) BS_VJPL(T, CP, false, false);                             \
+    else if (grad_w) BS_VJPL(T, CP, true, true);                        \
+    else BS_VJPL(T, CP, true, false);                                   \
+  } while (0)
+#define BS_VJPL3(T)                                                                         \
+  do {                                                                                      \
+    if (cpr == 1) BS_VJPL2(T, 1); else if (cpr == 2) BS_VJPL2(T, 2);                        \
+    else if (cpr <= 4) BS_VJPL2(T, 4); else if (cpr <= 8) BS_VJPL2(T, 8);                   \
+    else BS_VJPL2(T, 16);                                                                   \
+  } while (0)
+    if (spk_dtype == BS_SPK_U8) BS_VJPL3(uint8_t); else BS_VJPL3(float);
+#undef BS_VJPL3
+#undef BS_VJPL2
+#undef BS_VJPL
+    BS_CHECK_LAUNCH();
     return BS_OK;
   }
   const int g = grid_for(n_pre);
