@@ -223,10 +223,9 @@ __global__ __launch_bounds__(kBB) void k_bucket_qexp(const uint32_t* wmax, const
 
 // ---- step ----
 // 16 bytes of spikes (16 u8 rows or 4 f32 rows) of block blk = rows [blk*E, blk*E + E), rows
-// outside [r0, r1) read as 0: one vector load when the whole block lies inside and the
-// vector is 16-byte aligned, else one load per row in range.
-// The per-row form, out of line: it runs only for a block cut by the range or an unaligned
-// vector, and kept inline its code (in every load slot) would be fetched by the instruction
+// outside [r0, r1) read as 0: one vector load when the whole block lies inside (of any
+// alignment: a batch row of an odd length starts anywhere), else one load per row in range.
+// The per-row form, out of line: it runs only for a block cut by the range, and kept inline its code (in every load slot) would be fetched by the instruction
 // cache on every path (measured: 5x the misses of a compact kernel, ~2 us of a dense step).
 template <typename T>
 __device__ __noinline__ uint4 spike_block_rows(const T* __restrict__ spk, uint32_t row,
@@ -244,12 +243,16 @@ __device__ __noinline__ uint4 spike_block_rows(const T* __restrict__ spk, uint32
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-template <typename T, bool kVec>
+struct __attribute__((packed, aligned(1))) Any16 {
+  uint4 v;
+};
+
+template <typename T>
 __device__ __forceinline__ uint4 spike_block(const T* __restrict__ spk, uint32_t blk, uint32_t r0,
                                              uint32_t r1) {
   constexpr uint32_t kE = 16 / sizeof(T);
   const uint32_t row = blk * kE;  // rows < 2^31: 32-bit index math (a 64-bit op costs two)
-  if (kVec && row >= r0 && row + kE <= r1) return *(const uint4*)(spk + row);
+  if (row >= r0 && row + kE <= r1) return ((const Any16*)(spk + row))->v;
   return spike_block_rows<T>(spk, row, r0, r1);
 }
 
@@ -317,7 +320,7 @@ __device__ __forceinline__ void wave_prefix(uint32_t c, int& excl, int& total) {
 //   3. waves take kRowsPer rows at a time and issue the loads of up to kPasses 64-synapse
 //      passes of all of them before their LDS atomics;
 //   4. R_eff = 1: the bucket's outputs, with k_bucket_reduce's arithmetic; else partial r.
-template <typename T, bool kHet, bool kVec, bool kSingle>
+template <typename T, bool kHet, bool kSingle>
 __global__ __launch_bounds__(kSB) void k_bucket_scatter(
     const T* __restrict__ spk, int32_t n_pre, int32_t R, int32_t Rmax, int32_t nb, int32_t P,
     int32_t nsub,
@@ -335,6 +338,11 @@ __global__ __launch_bounds__(kSB) void k_bucket_scatter(
   __shared__ int32_t s_wave[2][kW];
   const int lane = bs_lane();
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / BS_WAVE));
+  // batch row blockIdx.y: its spikes, outputs, header and partials
+  spk += (int64_t)blockIdx.y * n_pre;
+  out += (int64_t)blockIdx.y * n_post;
+  hdr += blockIdx.y * (kHdr / 4);
+  part += (int64_t)blockIdx.y * R * n_post;
   // workgroup (b, sub, r): bucket b, sub-range sub of its posts (nsub > 1 only with R = 1),
   // row group r
   const int32_t b = blockIdx.x % nb;
@@ -405,7 +413,7 @@ __global__ __launch_bounds__(kSB) void k_bucket_scatter(
                                    : (r == 0 ? nblk : (specR ? (g1R + kE - 1) / kE : 0u));
     const uint32_t blk = first + threadIdx.x;
     const bool want = blk < lim;
-    v0[d] = want ? spike_block<T, kVec>(spk, blk, lo, hi) : make_uint4(0u, 0u, 0u, 0u);
+    v0[d] = want ? spike_block<T>(spk, blk, lo, hi) : make_uint4(0u, 0u, 0u, 0u);
   }
   // the bucket's LDS accumulator cleared while the loads are in flight (16-byte stores)
   // this workgroup's posts: [p0, p0 + pn), at offsets [lo_t, lo_t + pn) of bucket b
@@ -656,7 +664,7 @@ __global__ __launch_bounds__(kSB) void k_bucket_scatter(
 #pragma unroll
       for (int d = 0; d < kDepth; ++d) {
         const uint32_t blk = bb + (uint32_t)d * kSB + threadIdx.x;
-        v[d] = blk < bk1 ? spike_block<T, kVec>(spk, blk, g0, g1) : make_uint4(0u, 0u, 0u, 0u);
+        v[d] = blk < bk1 ? spike_block<T>(spk, blk, g0, g1) : make_uint4(0u, 0u, 0u, 0u);
       }
 #pragma unroll
       for (int d = 0; d < kDepth; ++d) mk[d] = spike_bits_sparse<T>(v[d]);
@@ -872,6 +880,9 @@ __global__ __launch_bounds__(256) void k_bucket_reduce(int32_t n_post, int32_t R
                                                        float* __restrict__ out) {
   const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (j >= n_post) return;
+  out += (int64_t)blockIdx.y * n_post;   // batch row
+  hdr += blockIdx.y * (kHdr / 4);
+  part += (int64_t)blockIdx.y * Rmax * n_post;
   constexpr int kFirst = 8;
   uint32_t x[kMaxR];   // the partials of j in row-group order (0 past R)
 #pragma unroll
@@ -918,6 +929,44 @@ int32_t row_groups(int32_t n_pre, int32_t nb) {
   if (R > rmax) R = rmax;
   if (R < 1) R = 1;
   return (int32_t)R;
+}
+
+// Row groups per batch row: a batch fills the chip with its own rows first.
+int32_t batch_row_groups(int32_t batch, int32_t n_pre, int32_t nb) {
+  const int64_t r = kTargetWgs / ((int64_t)nb * batch);
+  const int32_t rmax = row_groups(n_pre, nb);
+  return r < 1 ? 1 : (r < rmax ? (int32_t)r : rmax);
+}
+
+void scatter_launch(const void* spk, int32_t spk_dtype, int32_t batch, int32_t n_pre, int32_t R,
+                    int32_t Rmax, int32_t nb, int32_t P, int32_t nsub, bool single,
+                    const int32_t* seg, const uint16_t* lidx, const float* lw,
+                    const int32_t* qexp, int32_t n_post, float w_homo, int32_t accumulate,
+                    float* out, int32_t* hdr, int32_t* est_out, uint32_t* part, hipStream_t s) {
+  const dim3 g((unsigned)((int64_t)nb * nsub * R), (unsigned)batch);
+#define BS_BK1(T, H, SG)                                                                     \
+  k_bucket_scatter<T, H, SG><<<g, kSB, 0, s>>>((const T*)spk, n_pre, R, Rmax, nb, P, nsub, seg, \
+                                               lidx, lw, qexp, n_post, w_homo, accumulate,   \
+                                               out, hdr, est_out, part)
+#define BS_BK(T, H) do { if (single) BS_BK1(T, H, true); else BS_BK1(T, H, false); } while (0)
+  if (spk_dtype == BS_SPK_U8) { if (lw) BS_BK(uint8_t, true); else BS_BK(uint8_t, false); }
+  else { if (lw) BS_BK(float, true); else BS_BK(float, false); }
+#undef BS_BK
+#undef BS_BK1
+}
+
+int reduce_launch(int32_t batch, int32_t n_post, int32_t R, int32_t Rfix, const int32_t* hdr,
+                  const uint32_t* part, const float* lw, const int32_t* qexp, float w_homo,
+                  int32_t accumulate, float* out, hipStream_t s) {
+  const dim3 g((unsigned)(((int64_t)n_post + 255) / 256), (unsigned)batch);
+  if (lw)
+    k_bucket_reduce<true><<<g, 256, 0, s>>>(n_post, R, Rfix, hdr, part, qexp, w_homo, accumulate,
+                                            out);
+  else
+    k_bucket_reduce<false><<<g, 256, 0, s>>>(n_post, R, Rfix, hdr, part, qexp, w_homo, accumulate,
+                                             out);
+  BS_CHECK_LAUNCH();
+  return BS_OK;
 }
 
 int check_layout(int32_t n_pre, int32_t n_post, int32_t nb, int32_t P, const char* who) {
@@ -1050,46 +1099,72 @@ extern "C" int bs_event_bucket_f32(const void* spk, int32_t spk_dtype, int32_t n
                "bs_event_bucket_f32: workspace not 8-byte aligned");
   int32_t* hdr = (int32_t*)workspace;  // R_eff, written by the step kernel
   uint32_t* part = (uint32_t*)((char*)workspace + kHdr);
-  const int64_t g = (int64_t)nb * nsub * R;
-  const bool vec = (uintptr_t)spk % 16 == 0;  // 16-byte spike loads
-#define BS_BK(T, H, V)                                                                      \
-  do {                                                                                      \
-    if (single_launch)                                                                      \
-      k_bucket_scatter<T, H, V, true><<<(int)g, kSB, 0, s>>>(                               \
-          (const T*)spk, n_pre, R, Rmax, nb, P, nsub, seg, lidx, lw, qexp, n_post, w_homo,   \
-          accumulate, out, hdr, est_out, part);                                             \
-    else                                                                                    \
-      k_bucket_scatter<T, H, V, false><<<(int)g, kSB, 0, s>>>(                              \
-          (const T*)spk, n_pre, R, Rmax, nb, P, nsub, seg, lidx, lw, qexp, n_post, w_homo,   \
-          accumulate, out, hdr, est_out, part);                                             \
-  } while (0)
-#define BS_BK2(T, H) \
-  do { if (vec) BS_BK(T, H, true); else BS_BK(T, H, false); } while (0)
+  if (!dense) {
+    scatter_launch(spk, spk_dtype, 1, n_pre, R, Rmax, nb, P, nsub, single_launch, seg, lidx, lw,
+                   qexp, n_post, w_homo, accumulate, out, hdr, est_out, part, s);
+    BS_CHECK_LAUNCH();
+    if (single_launch) return BS_OK;
+    return reduce_launch(1, n_post, R, 0, hdr, part, lw, qexp, w_homo, accumulate, out, s);
+  }
+  const int64_t g = (int64_t)nb * R;
 #define BS_BD(T, H)                                                                         \
   k_bucket_scatter_dense<T, H><<<(int)g, kSB, 0, s>>>((const T*)spk, n_pre, rows, R, Rmax, nb, P, \
                                                       seg, lidx, lw, qexp, n_post, hdr, est_out, \
                                                       part)
-  if (dense) {
-    const int32_t rows = (int32_t)(((int64_t)n_pre + R - 1) / R);
-    if (spk_dtype == BS_SPK_U8) { if (lw) BS_BD(uint8_t, true); else BS_BD(uint8_t, false); }
-    else { if (lw) BS_BD(float, true); else BS_BD(float, false); }
-  } else if (spk_dtype == BS_SPK_U8) {
-    if (lw) BS_BK2(uint8_t, true); else BS_BK2(uint8_t, false);
-  } else {
-    if (lw) BS_BK2(float, true); else BS_BK2(float, false);
-  }
+  const int32_t rows = (int32_t)(((int64_t)n_pre + R - 1) / R);
+  if (spk_dtype == BS_SPK_U8) { if (lw) BS_BD(uint8_t, true); else BS_BD(uint8_t, false); }
+  else { if (lw) BS_BD(float, true); else BS_BD(float, false); }
 #undef BS_BD
-#undef BS_BK2
-#undef BS_BK
   BS_CHECK_LAUNCH();
-  if (single_launch) return BS_OK;
-  const int gr = (int)(((int64_t)n_post + 255) / 256);
-  if (lw)
-    k_bucket_reduce<true><<<gr, 256, 0, s>>>(n_post, R, dense ? R : 0, hdr, part, qexp, w_homo,
-                                             accumulate, out);
-  else
-    k_bucket_reduce<false><<<gr, 256, 0, s>>>(n_post, R, dense ? R : 0, hdr, part, qexp, w_homo,
-                                              accumulate, out);
+  return reduce_launch(1, n_post, R, R, hdr, part, lw, qexp, w_homo, accumulate, out, s);
+}
+
+extern "C" size_t bs_event_bucket_batch_workspace_size(int32_t batch, int32_t n_pre,
+                                                       int32_t n_post, int32_t nb) {
+  bs_clear_error();
+  if (batch <= 0 || n_pre <= 0 || n_post <= 0 || nb <= 0) return 0;
+  const int32_t R = batch_row_groups(batch, n_pre, nb);
+  return (size_t)batch * (kHdr + (R > 1 ? (size_t)R * n_post * sizeof(uint32_t) : 0));
+}
+
+extern "C" int bs_event_bucket_batch_f32(const void* spk, int32_t spk_dtype, int32_t batch,
+                                         int32_t n_pre, int32_t n_post, int32_t nb, int32_t P,
+                                         const int32_t* seg, const uint16_t* lidx,
+                                         const float* lw, const int32_t* qexp, float w_homo,
+                                         float* out, int32_t accumulate, void* workspace,
+                                         size_t workspace_bytes, bs_stream_t stream) {
+  bs_clear_error();
+  const char* fn = "bs_event_bucket_batch_f32";
+  int rc = check_layout(n_pre, n_post, nb, P, fn);
+  if (rc) return rc;
+  BS_CHECK_ARG(batch >= 0 && batch <= 65535, "%s: batch %d outside [0, 65535]", fn, batch);
+  BS_CHECK_ARG(spk_dtype == BS_SPK_U8 || spk_dtype == BS_SPK_F32, "%s: unknown spike dtype %d",
+               fn, spk_dtype);
+  if (batch == 0 || n_post == 0) return BS_OK;
+  BS_CHECK_ARG(out != nullptr, "%s: out is NULL", fn);
+  hipStream_t s = bs_stream(stream);
+  if (n_pre == 0) return accumulate ? BS_OK : bs_fill_f32(out, (int64_t)batch * n_post, 0.0f, s);
+  BS_CHECK_ARG(spk && seg && lidx, "%s: NULL pointer", fn);
+  BS_CHECK_ARG(spk_dtype == BS_SPK_U8 || (uintptr_t)spk % sizeof(float) == 0,
+               "%s: f32 spikes not 4-byte aligned", fn);
+  BS_CHECK_ARG(lw == nullptr || qexp != nullptr, "%s: qexp is NULL", fn);
+  const int32_t R = batch_row_groups(batch, n_pre, nb);
+  const size_t need = (size_t)batch * (kHdr + (R > 1 ? (size_t)R * n_post * sizeof(uint32_t) : 0));
+  BS_CHECK_ARG(workspace != nullptr && workspace_bytes >= need,
+               "%s: workspace of %zu bytes needed (got %zu)", fn, need,
+               workspace ? workspace_bytes : (size_t)0);
+  BS_CHECK_ARG((uintptr_t)workspace % 8 == 0, "%s: workspace not 8-byte aligned", fn);
+  int32_t* hdr = (int32_t*)workspace;  // one header per batch row, then the partials
+  uint32_t* part = (uint32_t*)((char*)workspace + (size_t)batch * kHdr);
+  int32_t nsub = 1;
+  if (R == 1) {
+    const int64_t per = kTargetWgs / ((int64_t)nb * batch);
+    nsub = (int32_t)(per < 1 ? 1 : (per > kSubSingle ? kSubSingle : per));
+    if (nsub > P) nsub = P;
+  }
+  scatter_launch(spk, spk_dtype, batch, n_pre, R, R, nb, P, nsub, R == 1, seg, lidx, lw, qexp,
+                 n_post, w_homo, accumulate, out, hdr, nullptr, part, s);
   BS_CHECK_LAUNCH();
-  return BS_OK;
+  if (R == 1) return BS_OK;
+  return reduce_launch(batch, n_post, R, 0, hdr, part, lw, qexp, w_homo, accumulate, out, s);
 }

@@ -332,11 +332,7 @@ class FixedNumConn(Module):
                 return ops.event_bucket(x, L)
             # [..., n_pre] spikes: each row through the bucketed operator (the same sums as a
             # replica inside the union runner)
-            rows = x.reshape(-1, x.shape[-1])
-            out = torch.empty(rows.shape[0], self.out_size[-1], dtype=torch.float32,
-                              device=x.device)
-            for b in range(rows.shape[0]):
-                ops.event_bucket(rows[b], L, out=out[b])
+            out = ops.event_bucket_batch(x.reshape(-1, x.shape[-1]), L)
             return out.reshape(tuple(x.shape[:-1]) + (self.out_size[-1],))
         conn = self.conn.with_data(w)
         return conn.matvec_events(x, value)   # [..., n_pre] -> [..., n_post], one launch

@@ -409,6 +409,37 @@ def event_bucket(spk, layout, out=None, accumulate=False, mode='auto'):
     return out
 
 
+def event_bucket_batch(spk, layout, out=None, accumulate=False):
+    """``event_bucket`` of every row of spk [B, n_pre] -> [B, n_post], each row with the bits
+    ``event_bucket`` gives it, in one or two launches for the whole batch."""
+    spk = _spk_view(spk)
+    L = layout
+    dev = L['seg'].device
+    B, n_pre = int(spk.shape[0]), L['n_pre']
+    if spk.shape[1] < n_pre:
+        raise ValueError(f'rows of {spk.shape[1]} spikes for {n_pre} pre rows')
+    if spk.shape[1] > n_pre:   # as event_bucket, which reads the leading n_pre
+        spk = spk[:, :n_pre].contiguous()
+    fixed = _bucket_call_args(L)[0]
+    if out is None:
+        out = torch.empty((B, L['n_post']), dtype=torch.float32, device=dev)
+    sh = torch.cuda.current_stream(dev).cuda_stream
+    key = ('bucket', dev.index, sh)
+    for b0 in range(0, B, 65535):
+        nb = min(65535, B - b0)
+        nbytes = int(N.lib().bs_event_bucket_batch_workspace_size(nb, n_pre, L['n_post'],
+                                                                  L['nb']))
+        ws = _WS_CACHE.get(key)
+        if nbytes > 0 and (ws is None or ws.numel() < nbytes):
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            _WS_CACHE[key] = ws
+        N.check(N.lib().bs_event_bucket_batch_f32(
+            N.ptr(spk[b0:b0 + nb]), _spk_dtype(spk), nb, *fixed, N.ptr(out[b0:b0 + nb]),
+            1 if accumulate else 0, N.ptr(ws) if nbytes > 0 else None, nbytes,
+            ctypes.c_void_p(sh)), 'bs_event_bucket_batch_f32')
+    return out
+
+
 def event_dense(spk, W, float_as_event=True, out=None):
     """spk [B, n_in] (or [n_in]) x W [n_in, n_out] -> [B, n_out]."""
     squeeze = spk.dim() == 1

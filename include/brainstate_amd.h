@@ -189,6 +189,18 @@ BS_API int bs_event_bucket_f32(const void* spk, int32_t spk_dtype, int32_t n_pre
                                int32_t accumulate, void* workspace, size_t workspace_bytes,
                                int32_t mode, int32_t* est_out, bs_stream_t stream);
 
+/* bs_event_bucket_f32 for `batch` spike rows spk [batch, n_pre] onto out [batch, n_post] in one
+ * or two launches: every row gets the bits bs_event_bucket_f32 gives it (any mode).  At most
+ * 65535 rows; the workspace needs bs_event_bucket_batch_workspace_size bytes. */
+BS_API size_t bs_event_bucket_batch_workspace_size(int32_t batch, int32_t n_pre, int32_t n_post,
+                                                   int32_t nb);
+BS_API int bs_event_bucket_batch_f32(const void* spk, int32_t spk_dtype, int32_t batch,
+                                     int32_t n_pre, int32_t n_post, int32_t nb, int32_t P,
+                                     const int32_t* seg, const uint16_t* lidx, const float* lw,
+                                     const int32_t* qexp, float w_homo, float* out,
+                                     int32_t accumulate, void* workspace,
+                                     size_t workspace_bytes, bs_stream_t stream);
+
 /* ---------------------------------------------------------------- N2b event gather
  * Same operator as N2a, post-major and deterministic (no atomics).  Spikes come as a
  * bitmap (bs_spike_pack: bit i%32 of word i/32 set <=> spk[i] != 0).  Layout SELL-64x4:

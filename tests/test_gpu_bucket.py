@@ -421,3 +421,36 @@ def test_bucket_graph_replays(torch_cuda):
         assert np.array_equal(out.cpu().numpy(), eager[j]), rep
         again = ops.event_bucket(spks[(j + 1) % 3], L).cpu().numpy()
         assert np.array_equal(again, eager[(j + 1) % 3])
+
+
+# rows of every alignment; one row group per batch row, several (small batches of long rows)
+# and posts split over workgroups (one short row); more active rows than a list holds
+@pytest.mark.parametrize('B,n_pre,n_post,k,p', [(64, 3200, 4000, 80, 0.02), (1, 333, 77, 5, 0.3),
+                                                (3, 20_001, 1500, 30, 0.3), (2, 9000, 30_001, 60, 0.9),
+                                                (130, 17, 9, 3, 0.5), (33, 4097, 13_000, 11, 1.0)])
+@pytest.mark.parametrize('het', [True, False])
+@pytest.mark.parametrize('sdt', ['u8', 'f32'])
+def test_bucket_batch_equals_rows(torch_cuda, B, n_pre, n_post, k, p, het, sdt):
+    torch = torch_cuda
+    from brainstate_amd import ops
+    say('bucket batch', B, n_pre, n_post, k, p, het, sdt)
+    rs = np.random.RandomState(B + k)
+    idx = dev(torch, rs.randint(-1, n_post + 1, (n_pre, k)).astype(np.int32))
+    w = dev(torch, rs.randn(n_pre, k).astype(np.float32)) if het else None
+    L = ops.build_buckets(idx, n_post, w=w, w_homo=0.3)
+    s = rs.rand(B, n_pre) < p
+    x = dev(torch, s.astype(np.uint8) if sdt == 'u8' else (s * rs.rand(B, n_pre)).astype(np.float32))
+    out = ops.event_bucket_batch(x, L)
+    acc = torch.ones(B, n_post, device='cuda')
+    ops.event_bucket_batch(x, L, out=acc, accumulate=True)
+    for b in range(B):
+        want = ops.event_bucket(x[b], L, mode='split')
+        assert torch.equal(out[b], want), b
+        if b < 3:
+            row = torch.ones(n_post, device='cuda')
+            ops.event_bucket(x[b], L, out=row, accumulate=True, mode='split')
+            assert torch.equal(acc[b], row), b
+    wide = torch.cat([x, x[:, :1]], 1)            # longer rows: their leading n_pre spikes
+    assert torch.equal(ops.event_bucket_batch(wide, L), out)
+    with pytest.raises(ValueError):
+        ops.event_bucket_batch(x[:, :-1], L)
