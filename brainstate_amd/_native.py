@@ -210,6 +210,16 @@ def ptr(t):
         return ctypes.c_void_p(t.data_ptr())
 
 
-def stream_handle(device=None):
+def raw_stream(device=None):
+    """The current stream of ``device`` (None: the current device) as an integer, without the
+    torch.cuda.Stream object (9 us of Python per call)."""
     import torch
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    index = None if device is None else device.index
+    if index is None:
+        index = torch.cuda.current_device()
+    get = getattr(torch._C, '_cuda_getCurrentRawStream', None)
+    return get(index) if get is not None else torch.cuda.current_stream(index).cuda_stream
+
+
+def stream_handle(device=None):
+    return ctypes.c_void_p(raw_stream(device))

@@ -25,6 +25,7 @@ Tensors live on the GPU; there is no CPU path.
 """
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from .. import _native as N
 from .. import ops
@@ -42,6 +43,9 @@ def _device():
 
 def _to_dev(a, dtype):
     if torch.is_tensor(a):
+        if a.is_cuda and a.dtype == dtype and a.is_contiguous() and \
+                a.device.index == torch.cuda.current_device():
+            return a
         return a.to(device=_device(), dtype=dtype).contiguous()
     return torch.as_tensor(np.ascontiguousarray(np.asarray(a)), dtype=dtype, device=_device())
 
@@ -66,6 +70,28 @@ def _grad_weight(w, like):
     return torch.tensor(float(w), dtype=torch.float32, device=like.device)
 
 
+def _record(fn, *args):
+    """Apply the autograd Function ``fn``.  torch binds the arguments of a Function with its own
+    ``setup_context`` to the forward's signature on every call (~30 us); outside torch.func
+    transforms, which need that form, the same Function with the context passed to
+    ``forward`` is applied instead (same saved tensors, ``backward`` and ``jvp``)."""
+    if torch._C._are_functorch_transforms_active():
+        return fn.apply(*args)
+    return fn._direct.apply(*args)
+
+
+def _with_direct(fn):
+    def forward(ctx, *args):
+        out = fn.forward(*args)
+        fn.setup_context(ctx, args, out)
+        return out
+    fn._direct = type(fn.__name__ + 'Direct', (torch.autograd.Function,), {
+        'forward': staticmethod(forward), 'backward': staticmethod(fn.backward),
+        'jvp': staticmethod(fn.jvp), '__module__': fn.__module__})
+    return fn
+
+
+@_with_direct
 class _EventMatvecFn(torch.autograd.Function):
     """out = mat-vec of spk with weights w over (indices, indptr): every nonzero spike is one
     event (value=False) or weighs by its value (value=True).  Differentiable in the spike
@@ -121,7 +147,6 @@ class _EventMatvecFn(torch.autograd.Function):
 def _no_autodiff(*ts):
     """True when no operand takes part in reverse or forward mode autodiff (including the
     wrapped tensors of torch.func transforms)."""
-    from torch.autograd import forward_ad
     for t in ts:
         if torch.is_tensor(t):
             if t.requires_grad and torch.is_grad_enabled():
@@ -165,8 +190,8 @@ class FixedPostNumConn:
         if torch.is_tensor(w) and w.numel() > 1:
             w = w.expand(self.indices.shape) if w.shape != self.indices.shape else w
         if _wants_grad(spk, w):
-            return _EventMatvecFn.apply(spk, _grad_weight(w, spk), self.indices, None, n_post,
-                                        value)
+            return _record(_EventMatvecFn, spk, _grad_weight(w, spk), self.indices, None, n_post,
+                           value)
         wk = _kw(w) if torch.is_tensor(w) else w
         if value:
             return ops.value_matvec(spk, self.indices, wk, n_post)
@@ -190,8 +215,8 @@ class CSR:
         if torch.is_tensor(w) and w.numel() > 1 and w.shape != self.indices.shape:
             w = w.expand(self.indices.shape)
         if _wants_grad(spk, w):
-            return _EventMatvecFn.apply(spk, _grad_weight(w, spk), self.indices, self.indptr,
-                                        n_post, value)
+            return _record(_EventMatvecFn, spk, _grad_weight(w, spk), self.indices, self.indptr,
+                           n_post, value)
         wk = _kw(w) if torch.is_tensor(w) else w
         if value:
             return ops.value_matvec(spk, self.indices, wk, n_post, indptr=self.indptr)
@@ -404,6 +429,7 @@ class EventFixedNumConn(FixedNumConn):
 EventFixedProb = EventFixedNumConn
 
 
+@_with_direct
 class _EventDenseFn(torch.autograd.Function):
     """out = spk @ W (rows of W selected by the nonzero spikes when float_as_event, else
     weighted by the spike values); derivatives of spk_values @ W in both modes."""
@@ -440,6 +466,7 @@ class _EventDenseFn(torch.autograd.Function):
         return t
 
 
+@_with_direct
 class _HomoLinearFn(torch.autograd.Function):
     """EventLinear's homogeneous shortcut (brainstate/nn/_event_linear.py:77-97): every output
     is (count of nonzero spikes, or their sum) * w.  Derivatives of x @ (ones * w), as the
@@ -538,19 +565,21 @@ class EventLinear(Module):
         x = spk if torch.is_tensor(spk) else _to_dev(spk, torch.float32)
         if x.device.type != 'cuda':
             x = x.to(_device())
-        n_w = 1 if init._is_scalar(w) else int(np.prod(w.shape))
+        n_w = 1 if init._is_scalar(w) else (w.numel() if torch.is_tensor(w) else int(np.prod(w.shape)))
         if n_w == 1:
             # homogeneous shortcut, :77-97 (reference-owned arithmetic on the reduction)
             wt = _grad_weight(_weight_for_kernel(w), x).reshape(())
-            return _HomoLinearFn.apply(x, wt, self.out_size[-1], self.float_as_event)
+            return _record(_HomoLinearFn, x, wt, self.out_size[-1], self.float_as_event)
         W = _module_weight(self, w)
-        W = W.expand(self.in_size[-1], self.out_size[-1]).contiguous()
+        if tuple(W.shape) != (self.in_size[-1], self.out_size[-1]):
+            W = W.expand(self.in_size[-1], self.out_size[-1])
+        W = W.contiguous()
         if x.dtype not in (torch.bool, torch.uint8, torch.float32):
             x = x.to(torch.float32)
         if _no_autodiff(x, W):
             P = self._packed_weight(W)
             if P is not None:
                 return ops.event_dense_packed(x, P)
-        if _wants_grad(x, W):
-            return _EventDenseFn.apply(x, W, self.float_as_event)
+        elif torch.is_grad_enabled():
+            return _record(_EventDenseFn, x, W, self.float_as_event)
         return ops.event_dense(x, W, float_as_event=self.float_as_event)

@@ -4,6 +4,8 @@ These are the building blocks the brainstate-compatible layers call; each maps o
 C entry point of include/brainstate_amd.h and raises ``NativeError`` on failure.
 """
 import ctypes
+import functools
+import math
 
 import numpy as np
 import torch
@@ -31,7 +33,7 @@ def _spk_view(spk):
 def compact_workspace(n, device):
     """Zero-filled workspace for bs_spike_compact, cached per (device, stream, size)."""
     nbytes = int(N.lib().bs_spike_compact_workspace_size(int(n)))
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, N.raw_stream(device))
     ws = _WS_CACHE.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.zeros(max(nbytes, 4096), dtype=torch.uint8, device=device)
@@ -75,7 +77,7 @@ def event_scatter(active, n_active, indices, w, n_post, k=None, indptr=None, out
 def _batch_of(x):
     """(leading shape, batch rows, row length) of a [..., n] operand."""
     lead = tuple(x.shape[:-1])
-    return lead, int(np.prod(lead)) if lead else 1, int(x.shape[-1]) if x.dim() else 1
+    return lead, math.prod(lead), int(x.shape[-1]) if x.dim() else 1
 
 
 def event_matvec(spk, indices, w, n_post, k=None, indptr=None, out=None, accumulate=False):
@@ -396,7 +398,7 @@ def event_bucket(spk, layout, out=None, accumulate=False, mode='auto'):
                          f"got {mode!r}")
     if out is None:
         out = torch.empty(L['n_post'], dtype=torch.float32, device=dev)
-    sh = torch.cuda.current_stream(dev).cuda_stream
+    sh = N.raw_stream(dev)
     key = ('bucket', dev.index, sh)
     ws = _WS_CACHE.get(key)
     if nbytes > 0 and (ws is None or ws.numel() < nbytes):
@@ -423,7 +425,7 @@ def event_bucket_batch(spk, layout, out=None, accumulate=False):
     fixed = _bucket_call_args(L)[0]
     if out is None:
         out = torch.empty((B, L['n_post']), dtype=torch.float32, device=dev)
-    sh = torch.cuda.current_stream(dev).cuda_stream
+    sh = N.raw_stream(dev)
     key = ('bucket', dev.index, sh)
     for b0 in range(0, B, 65535):
         nb = min(65535, B - b0)
@@ -440,6 +442,13 @@ def event_bucket_batch(spk, layout, out=None, accumulate=False):
     return out
 
 
+@functools.lru_cache(maxsize=256)
+def _dense_ws(B, n_in, n_out):
+    """(workspace bytes, ticket bytes) of bs_event_dense_f32: functions of the shape alone."""
+    return (int(N.lib().bs_event_dense_workspace_size(B, n_in, n_out)),
+            int(N.lib().bs_event_dense_ticket_bytes(B, n_in, n_out)))
+
+
 def event_dense(spk, W, float_as_event=True, out=None):
     """spk [B, n_in] (or [n_in]) x W [n_in, n_out] -> [B, n_out]."""
     squeeze = spk.dim() == 1
@@ -448,14 +457,13 @@ def event_dense(spk, W, float_as_event=True, out=None):
     n_out = W.shape[1]
     if out is None:
         out = torch.empty(B, n_out, dtype=torch.float32, device=W.device)
-    nbytes = int(N.lib().bs_event_dense_workspace_size(B, n_in, n_out))
+    nbytes, tick = _dense_ws(B, n_in, n_out)
     ws = None
     if nbytes > 0:
         # ticket counters lead the workspace: zero on entry, left zero by every call; the
         # bytes after them hold partial sums, so bytes past the previous call's counters
         # are zeroed before a call that needs more counters
-        tick = int(N.lib().bs_event_dense_ticket_bytes(B, n_in, n_out))
-        key = ('dense', W.device.index, torch.cuda.current_stream(W.device).cuda_stream)
+        key = ('dense', W.device.index, N.raw_stream(W.device))
         ws, zero = _WS_CACHE.get(key, (None, 0))
         if ws is None or ws.numel() < nbytes:
             ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=W.device)
