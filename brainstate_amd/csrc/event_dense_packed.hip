@@ -193,40 +193,54 @@ __device__ __forceinline__ uint32_t nz_bytes(uint32_t x) {
   return ((((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) >> 7) & 0x01010101u;
 }
 
+// 16 bytes at any address.
+struct __attribute__((packed, aligned(1))) Any16 {
+  v4i v;
+};
+
+// How the spikes are read: 16 inputs of a lane at a time when n_in >= 16, at any alignment,
+// from an address clamped into the row.  When n_in is not a multiple of 16 (kCut), the lane
+// that holds the row's end then has its 16 inputs kCutBy = 16 - n_in % 16 bytes late
+// (cut_shift); inputs at or past n_in meet zero digits, so what they read does not matter.
+enum SpkRead { kSlow, kWide, kCut };
+
+// x moved down by d bytes (d uniform, 1 .. 15).
+__device__ __forceinline__ v4i cut_shift(v4i x, int d) {
+  const int w = d >> 2;
+  v4i y;
+  y[0] = w == 0 ? x[0] : w == 1 ? x[1] : w == 2 ? x[2] : x[3];
+  y[1] = w == 0 ? x[1] : w == 1 ? x[2] : x[3];
+  y[2] = w == 0 ? x[2] : x[3];
+  y[3] = x[3];
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    y[q] = (int32_t)__builtin_amdgcn_alignbyte((uint32_t)y[q < 3 ? q + 1 : 3], (uint32_t)y[q],
+                                               (uint32_t)(d & 3));
+  return y;
+}
+
 // Spike operand of one row tile for input block k: lane holds batch row b, inputs
 // 64 k + 16 (lane / 16) + [0, 16) as 0/1 bytes.
-template <typename T, bool kVec>
+template <typename T, SpkRead kRead>
 __device__ __forceinline__ v4i load_spk(const T* __restrict__ spk, int32_t batch, int32_t n_in,
                                         int32_t b, int64_t i0) {
   v4i a = {0, 0, 0, 0};
+  if constexpr (sizeof(T) == 4 && kRead != kSlow) {
+    const T* p = spk + (int64_t)(b < batch ? b : batch - 1) * n_in +
+                 (i0 + 16 <= n_in ? i0 : (int64_t)n_in - 16);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const v4i x = ((const Any16*)(p + 4 * q))->v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[q] |= (x[e] & 0x7fffffff) != 0 ? 1 << (8 * e) : 0;
+    }
+    return a;
+  }
   if (b >= batch || i0 >= n_in) return a;
   const T* p = spk + (int64_t)b * n_in + i0;
-  if constexpr (sizeof(T) == 1) {
-    if (kVec) {  // n_in % 16 == 0 and 16-byte aligned rows: i0 + 16 <= n_in
-      const uint4 x = *(const uint4*)p;
-      a[0] = (int32_t)nz_bytes(x.x);
-      a[1] = (int32_t)nz_bytes(x.y);
-      a[2] = (int32_t)nz_bytes(x.z);
-      a[3] = (int32_t)nz_bytes(x.w);
-    } else {
 #pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (i0 + u < n_in && p[u] != 0) a[u >> 2] |= 1 << (8 * (u & 3));
-    }
-  } else {
-    if (kVec) {  // n_in % 16 == 0 and 16-byte aligned rows
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float4 x = *(const float4*)(p + 4 * q);
-        a[q] = (x.x != 0.0f ? 1 : 0) | (x.y != 0.0f ? 1 << 8 : 0) |
-               (x.z != 0.0f ? 1 << 16 : 0) | (x.w != 0.0f ? 1 << 24 : 0);
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (i0 + u < n_in && p[u] != 0.0f) a[u >> 2] |= 1 << (8 * (u & 3));
-    }
-  }
+  for (int u = 0; u < 16; ++u)
+    if (i0 + u < n_in && p[u] != T(0)) a[u >> 2] |= 1 << (8 * (u & 3));
   return a;
 }
 
@@ -241,7 +255,7 @@ struct LifOut {
   bs_lif_params p;
 };
 
-template <typename T, int L, bool kVec, bool kLif>
+template <typename T, int L, SpkRead kRead, bool kLif>
 __global__ __launch_bounds__(kPB) void k_event_dense_packed(
     const T* __restrict__ spk, int32_t batch, int32_t n_in, const uint8_t* __restrict__ dig,
     const uint32_t* __restrict__ bits, const uint32_t* __restrict__ status, int32_t n_out,
@@ -293,9 +307,12 @@ __global__ __launch_bounds__(kPB) void k_event_dense_packed(
   // one pipeline stage: kGroup input blocks.  Every wave's block range is whole stages (KB is
   // a multiple of kPW * kGroup), so no stage reaches past it.  Byte spikes on the 16-byte path
   // are loaded from clamped addresses (rows past `batch` repeat the last row, whose sums are
-  // never stored; inputs past n_in repeat the last 16, whose digits are zero), kept raw and
+  // never stored; inputs past n_in read the row's last 16, and meet zero digits), kept raw and
   // masked when multiplied, so the loads need no masks or branches and none waits for another.
-  constexpr bool kRaw = sizeof(T) == 1 && kVec;
+  // 100 x 1000 spikes, 1000 x 300 W: 28 us with a byte at a time (rows not 16-byte aligned), 6
+  // this way.
+  constexpr bool kRaw = sizeof(T) == 1 && kRead != kSlow;
+  const int cut = n_in & 15;                          // inputs of the lane at the row's end
   auto load = [&](int32_t k, v4i (&a)[kGroup][kRowTiles], v4i (&bv)[kGroup][L]) {
 #pragma unroll
     for (int s = 0; s < kGroup; ++s) {
@@ -308,20 +325,27 @@ __global__ __launch_bounds__(kPB) void k_event_dense_packed(
         const int32_t b = brow + 16 * mt;
         if constexpr (kRaw) {
           const int64_t off = (int64_t)(b < batch ? b : batch - 1) * n_in +
-                              (i0 < n_in ? i0 : (int64_t)n_in - 16);
-          a[s][mt] = *(const v4i*)((const uint8_t*)spk + off);
+                              (i0 + 16 <= n_in ? i0 : (int64_t)n_in - 16);
+          a[s][mt] = ((const Any16*)((const uint8_t*)spk + off))->v;
         } else {
-          a[s][mt] = load_spk<T, kVec>(spk, batch, n_in, b, i0);
+          a[s][mt] = load_spk<T, kRead>(spk, batch, n_in, b, i0);
         }
       }
     }
   };
-  auto mult = [&](const v4i (&a)[kGroup][kRowTiles], const v4i (&bv)[kGroup][L]) {
+  auto mult = [&](int32_t k, const v4i (&a)[kGroup][kRowTiles], const v4i (&bv)[kGroup][L]) {
 #pragma unroll
     for (int s = 0; s < kGroup; ++s)
 #pragma unroll
       for (int mt = 0; mt < kRowTiles; ++mt) {
         v4i x = a[s][mt];
+        if constexpr (kRead == kCut) {
+          if (k + s == n_in / kBlkIn) {               // uniform: the block with the row's end
+            const v4i y = cut_shift(x, 16 - cut);
+            const int64_t i0 = (int64_t)(k + s) * kBlkIn + iq;
+            if (i0 < n_in && i0 + 16 > n_in) x = y;
+          }
+        }
         if constexpr (kRaw) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) x[q] = (int32_t)nz_bytes((uint32_t)x[q]);
@@ -344,16 +368,16 @@ __global__ __launch_bounds__(kPB) void k_event_dense_packed(
     int32_t k = k_lo;
     for (; k + 2 * kGroup < k_hi; k += 2 * kGroup) {
       sched(); load(k + kGroup, a1, b1v); sched();
-      mult(a0, b0v);
+      mult(k, a0, b0v);
       sched(); load(k + 2 * kGroup, a0, b0v); sched();
-      mult(a1, b1v);
+      mult(k + kGroup, a1, b1v);
     }
     if (k + kGroup < k_hi) {
       sched(); load(k + kGroup, a1, b1v); sched();
-      mult(a0, b0v);
-      mult(a1, b1v);
+      mult(k, a0, b0v);
+      mult(k + kGroup, a1, b1v);
     } else {
-      mult(a0, b0v);
+      mult(k, a0, b0v);
     }
   }
 
@@ -401,7 +425,7 @@ __global__ __launch_bounds__(kPB) void k_event_dense_packed(
 
 template <typename T, int L>
 void launch_packed(const T* spk, int32_t batch, int32_t n_in, const PackDims& d,
-                   const uint8_t* packed, int32_t n_out, float* out, bool vec,
+                   const uint8_t* packed, int32_t n_out, float* out, SpkRead rd,
                    const LifOut* lif, hipStream_t s) {
   const dim3 grid(d.NT, (batch + kGroupB - 1) / kGroupB);
   const uint8_t* dig = packed + d.dig_off;
@@ -411,8 +435,14 @@ void launch_packed(const T* spk, int32_t batch, int32_t n_in, const PackDims& d,
 #define BS_PK(V, F)                                                                        \
   k_event_dense_packed<T, L, V, F><<<grid, kPB, 0, s>>>(spk, batch, n_in, dig, bits, status, \
                                                         n_out, d.KB, out, F ? *lif : none)
-  if (lif) { if (vec) BS_PK(true, true); else BS_PK(false, true); }
-  else { if (vec) BS_PK(true, false); else BS_PK(false, false); }
+#define BS_PK2(F)                                                   \
+  do {                                                              \
+    if (rd == kWide) BS_PK(kWide, F);                               \
+    else if (rd == kCut) BS_PK(kCut, F);                            \
+    else BS_PK(kSlow, F);                                           \
+  } while (0)
+  if (lif) BS_PK2(true); else BS_PK2(false);
+#undef BS_PK2
 #undef BS_PK
 }
 
@@ -432,8 +462,7 @@ int packed_product(const char* fn, const void* spk, int32_t spk_dtype, int32_t b
   BS_CHECK_ARG(spk != nullptr || n_in == 0, "%s: spk is NULL", fn);
   const PackDims d = pack_dims(n_in, n_out);
   const uint8_t* pk = (const uint8_t*)packed;
-  const size_t es = spk_dtype == BS_SPK_U8 ? 1 : 4;
-  const bool vec = n_in % 16 == 0 && ((uintptr_t)spk & 15) == 0 && (n_in * es) % 16 == 0;
+  const SpkRead vec = n_in < 16 ? kSlow : n_in % 16 == 0 ? kWide : kCut;
   if (spk_dtype == BS_SPK_U8) {
     const uint8_t* p = (const uint8_t*)spk;
     switch (d.L) {

@@ -273,3 +273,26 @@ def test_packed_lif_step_rejects_overlapping_outputs(torch_cuda):
     out = torch.empty(B, n, dtype=torch.uint8, device='cuda')
     ops.event_dense_packed_lif_step(buf, P, V, ge, gi, ref, ops.lif_params(), spk_out=out)
     torch.cuda.synchronize()
+
+
+# rows that end in every position of a 16-input group, in the first and the last input block of
+# a wave, one input group long, and rows starting at odd addresses
+@pytest.mark.parametrize('n_in', [15, 16, 17, 31, 33, 63, 79, 497, 1000, 1023, 2051])
+@pytest.mark.parametrize('sdt', ['u8', 'f32'])
+def test_packed_ragged_rows(torch_cuda, n_in, sdt):
+    torch = torch_cuda
+    from brainstate_amd import ops
+    say('packed ragged', n_in, sdt)
+    rng = np.random.RandomState(n_in)
+    B, n_out = 70, 37
+    W = rng.normal(0, 0.125, (n_in, n_out)).astype(F)
+    s = rng.rand(B, n_in) < 0.4
+    spk = (s * rng.randint(1, 256, (B, n_in))).astype(np.uint8) if sdt == 'u8' else \
+        np.where(s, -1.5, -0.0).astype(F)
+    P, got = run(torch, spk, W)
+    want = event.event_dense_fixed_point(spk, W)
+    assert np.array_equal(got, want)
+    flat = dev(torch, np.concatenate([[1], spk.reshape(-1)]).astype(spk.dtype))
+    view = flat[1:].reshape(B, n_in)                # one element past a 16-byte boundary
+    assert np.array_equal(ops.event_dense_packed(view, P).cpu().numpy(), want)
+    assert np.array_equal(ops.event_dense_packed(view[-1], P).cpu().numpy(), want[-1])
