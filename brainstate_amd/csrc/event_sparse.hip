@@ -631,6 +631,188 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp_batch(
   }
 }
 
+// ---- the same with g transposed: gT[j][b], Bp columns (a multiple of LB), row n_post zero ----
+// A 4-byte gather of g moves a line for each (synapse, batch row); transposed, the batch values
+// of a synapse's target lie side by side.
+constexpr int kTr = 64;   // tile of the transposition
+__global__ __launch_bounds__(kBlock) void k_transpose_g(const float* __restrict__ g, int32_t batch,
+                                                        int32_t n_post, int32_t Bp,
+                                                        float* __restrict__ gT,
+                                                        uint32_t* __restrict__ odd) {
+  __shared__ float s_t[kTr][kTr + 1];
+  __shared__ uint32_t s_odd;
+  const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
+  const int64_t j0 = (int64_t)blockIdx.x * kTr, b0 = (int64_t)blockIdx.y * kTr;
+  if (threadIdx.x == 0) s_odd = 0u;
+  __syncthreads();
+  bool bad = false;
+#pragma unroll
+  for (int r = r0; r < kTr; r += kBlock / 64) {
+    const int64_t b = b0 + r, j = j0 + c;
+    const float v = b < batch && j < n_post ? g[b * n_post + j] : 0.0f;
+    bad |= (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u;
+    s_t[r][c] = v;
+  }
+  if (bad) s_odd = 1u;
+  __syncthreads();
+#pragma unroll
+  for (int r = r0; r < kTr; r += kBlock / 64) {
+    const int64_t j = j0 + r, b = b0 + c;
+    if (j <= n_post && b < Bp) gT[j * Bp + b] = s_t[c][r];
+  }
+  if (threadIdx.x == 0) odd[blockIdx.y * gridDim.x + blockIdx.x] = s_odd;  // inf or NaN in it
+}
+
+// One wave per pre row i.
+//   grad_x[b, i]: lane (q, b) = (lane / LB, lane % LB) sums the row's synapses l = a G + q of
+//   every 64 (G = 64 / LB) into its own accumulator a -- the lane sums of k_matvec_vjp, held
+//   by a instead of by lane -- and adds them in k_matvec_vjp's order: bit for bit its value.
+//   grad_w[i, k]: lane = synapse, the products x[b, i] g[b, idx] added in b order over the
+//   batch rows whose x is not zero (the others add +-0; unless some g is inf or NaN, `odd`:
+//   then over all).
+// 64 rows of 3200 -> 4000, K = 80: 101 us with per-row 4-byte gathers of g for both, 16 (and 7
+// for the transposition) here; bound by latency at that size, by L2 at 128 x 10k.
+template <typename T, bool kCsr, bool kHet, int LB>
+__global__ __launch_bounds__(kBlock) void k_matvec_vjp_bt(
+    const T* __restrict__ spk, int32_t batch, int32_t n_pre, const int32_t* __restrict__ indptr,
+    const int32_t* __restrict__ indices, int32_t k, const float* __restrict__ w, float w_homo,
+    int32_t n_post, const float* __restrict__ g, const float* __restrict__ gT, int32_t Bp,
+    const uint32_t* __restrict__ odd, int32_t n_odd, float* __restrict__ gx,
+    float* __restrict__ gw) {
+  constexpr int G = BS_WAVE / LB, A = LB, kU = 16;
+  const int lane = bs_lane();
+  const int q = lane / LB, bl = lane % LB;
+  const int64_t nw = (int64_t)gridDim.x * (kBlock / BS_WAVE);
+  const int32_t nnz = kCsr ? indptr[n_pre] : 0;
+  bool all = false;
+  if (kHet && gw)
+    for (int32_t t = lane; t < n_odd; t += BS_WAVE) all |= odd[t] != 0u;
+  all = bs_ballot(all) != 0ull;
+  float sw = 0.0f;
+  for (int64_t row = __builtin_amdgcn_readfirstlane(
+           (int)(((int64_t)blockIdx.x * kBlock + threadIdx.x) / BS_WAVE));
+       row < n_pre; row += nw) {
+    int64_t beg, end;
+    if (kCsr) {
+      beg = indptr[row];
+      end = indptr[row + 1];
+      beg = beg < 0 ? 0 : beg;
+      end = end > nnz ? nnz : end;
+    } else {
+      beg = row * k;
+      end = beg + k;
+    }
+    if (gx || !kHet) {
+      for (int32_t b0 = 0; b0 < batch; b0 += LB) {
+        const int32_t b = b0 + bl;
+        const float* gb = gT + b;                      // b < Bp
+        float acc[A], tot = 0.0f;
+#pragma unroll
+        for (int a = 0; a < A; ++a) acc[a] = 0.0f;
+        for (int64_t s0 = beg; s0 < end; s0 += BS_WAVE) {
+          const int cnt = (int)(end - s0 < BS_WAVE ? end - s0 : BS_WAVE);
+          const bool in = lane < cnt;
+          const int32_t js = in ? indices[s0 + lane] : n_post;
+          const int32_t jl = (uint32_t)js < (uint32_t)n_post ? js : n_post;   // the zero row
+          const float wl = !in ? 0.0f : (kHet ? w[s0 + lane] : w_homo);
+#pragma unroll
+          for (int a0 = 0; a0 < A; a0 += kU) {
+            if (a0 * G >= cnt) break;                  // uniform
+            float v[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+              const int l = (a0 + u) * G;
+              const int32_t j = G == 1 ? __builtin_amdgcn_readlane(jl, l) : __shfl(jl, l + q);
+              v[u] = gb[(uint32_t)j * (uint32_t)Bp];
+            }
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+              const int l = (a0 + u) * G;
+              const float ws = G == 1 ? __uint_as_float(__builtin_amdgcn_readlane(
+                                            __float_as_uint(wl), l))
+                                      : __shfl(wl, l + q);
+              acc[a0 + u] += ws * v[u];
+              if (!kHet) tot += v[u];
+            }
+          }
+        }
+#pragma unroll
+        for (int o = A / 2; o > 0; o >>= 1)
+#pragma unroll
+          for (int a = 0; a < o; ++a) acc[a] += acc[a + o];
+        float sx = acc[0];
+#pragma unroll
+        for (int o = BS_WAVE / 2; o >= LB; o >>= 1) sx += __shfl_xor(sx, o);
+        if (b < batch) {
+          if (gx && q == 0) gx[(int64_t)b * n_pre + row] = sx;
+          if (!kHet && gw) {
+            const float xv = (float)spk[(int64_t)b * n_pre + row];
+            if (xv != 0.0f) sw += xv * tot;            // this lane's share of the row's g
+          }
+        }
+      }
+    }
+    if (kHet && gw) {
+      for (int64_t s = beg + lane; s - lane < end; s += BS_WAVE) {
+        const int32_t js = s < end ? indices[s] : n_post;
+        const float* gj = gT + (uint32_t)((uint32_t)js < (uint32_t)n_post ? js : n_post) *
+                                   (uint32_t)Bp;
+        float acc = 0.0f;
+        for (int32_t b0 = 0; b0 < batch; b0 += BS_WAVE) {
+          const int32_t bx = b0 + lane;
+          const float xl = bx < batch ? (float)spk[(int64_t)bx * n_pre + row] : 0.0f;
+          uint64_t m = bs_ballot(bx < batch && (all || xl != 0.0f));
+          // kF values in flight (a row has a few active batch rows: one at a time, their
+          // latencies add up); past the last one the lowest is read again and not added
+          while (m) {
+            constexpr int kF = 8;
+            int at[kF];
+            bool on[kF];
+            float v[kF];
+            const int first = __builtin_ctzll(m);
+#pragma unroll
+            for (int f = 0; f < kF; ++f) {
+              on[f] = m != 0ull;
+              at[f] = on[f] ? __builtin_ctzll(m) : first;
+              m &= m - 1;
+              v[f] = gj[b0 + at[f]];
+            }
+#pragma unroll
+            for (int f = 0; f < kF; ++f) {
+              const float xv =
+                  __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(xl), at[f]));
+              const float prod = xv * v[f];
+              acc = on[f] ? acc + prod : acc;
+            }
+          }
+        }
+        if (s < end) gw[s] = acc;
+      }
+    }
+  }
+  if (!kHet && gw) {
+#pragma unroll
+    for (int o = BS_WAVE / 2; o > 0; o >>= 1) sw += __shfl_xor(sw, o);
+    block_atomic_sum<kBlock / BS_WAVE>(sw, gw);
+  }
+}
+
+int32_t vjp_lanes(int32_t batch) { return batch <= 16 ? 16 : 64; }
+
+// Workspace of the transposed form, 0 where the per-row form is kept: its extra launch costs
+// ~4 us, which a few batch rows of a small layer do not repay (us per call, per-row /
+// transposed: 2 x 3200 rows of 80 12.6 / 14.6, 3 x 500 of 500 13.2 / 17.4, 4 x 3200 of 80
+// 12.3 / 15.4, 8 x 10k of 100 55 / 19, 100 x 500 of 20 87 / 15, 128 x 10k of 100 1020 / 115).
+size_t vjp_bt_bytes(int32_t batch, int32_t n_pre, int32_t n_post) {
+  if (n_pre < 1 || n_post < 1 || batch < 3 || (batch < 8 && (int64_t)batch * n_pre < 20000))
+    return 0;
+  const int64_t Bp = ((int64_t)batch + vjp_lanes(batch) - 1) / vjp_lanes(batch) * vjp_lanes(batch);
+  const int64_t n = ((int64_t)n_post + 1) * Bp;
+  if (n >= (1LL << 30)) return 0;                      // 32-bit element offsets
+  const int64_t tiles = ((int64_t)n_post + kTr) / kTr * ((Bp + kTr - 1) / kTr);
+  return (size_t)(n + tiles) * 4;
+}
+
 int grid_for(int64_t work_items_waves) {
   const int64_t cap = (int64_t)bs_num_cus() * 16;
   int64_t b = (work_items_waves + (kBlock / BS_WAVE) - 1) / (kBlock / BS_WAVE);
@@ -823,13 +1005,12 @@ extern "C" int bs_value_matvec_batch_f32(const float* x, int32_t batch, int32_t 
                              out, accumulate, bs_stream(stream), "bs_value_matvec_batch_f32");
 }
 
-extern "C" int bs_event_matvec_vjp_batch_f32(const void* spk, int32_t spk_dtype, int32_t batch,
-                                             int32_t n_pre, const int32_t* indptr,
-                                             const int32_t* indices, int32_t k, const float* w,
-                                             float w_homo, int32_t n_post, const float* grad_out,
-                                             float* grad_spk, float* grad_w,
-                                             bs_stream_t stream) {
-  bs_clear_error();
+namespace {
+
+int vjp_batch(const void* spk, int32_t spk_dtype, int32_t batch, int32_t n_pre,
+              const int32_t* indptr, const int32_t* indices, int32_t k, const float* w,
+              float w_homo, int32_t n_post, const float* grad_out, float* grad_spk,
+              float* grad_w, void* ws, size_t ws_bytes, bs_stream_t stream) {
   BS_CHECK_ARG(batch >= 0 && n_pre >= 0 && n_post >= 0,
                "bs_event_matvec_vjp_batch_f32: negative size");
   BS_CHECK_ARG(indptr != nullptr || k >= 0, "bs_event_matvec_vjp_batch_f32: k=%d < 0", k);
@@ -847,8 +1028,36 @@ extern "C" int bs_event_matvec_vjp_batch_f32(const void* spk, int32_t spk_dtype,
   if (!csr && k == 0) {  // no synapse: grad_spk is zero, grad_w empty
     return grad_spk ? bs_fill_f32(grad_spk, (int64_t)batch * n_pre, 0.0f, s) : BS_OK;
   }
-  // batch == 0 or n_post == 0 go through the kernel: it writes grad_w = 0 (g never read)
   const int g = grid_for(n_pre);
+  const size_t need = vjp_bt_bytes(batch, n_pre, n_post);
+  if (need > 0 && ws != nullptr) {
+    BS_CHECK_ARG(ws_bytes >= need, "bs_event_matvec_vjp_batch_ws_f32: workspace of %zu bytes "
+                 "needed (got %zu)", need, ws_bytes);
+    const int32_t lanes = vjp_lanes(batch);
+    const int32_t Bp = (batch + lanes - 1) / lanes * lanes;
+    float* gT = (float*)ws;
+    uint32_t* odd = (uint32_t*)(gT + ((int64_t)n_post + 1) * Bp);
+    const dim3 tg((unsigned)(((int64_t)n_post + kTr) / kTr), (unsigned)((Bp + kTr - 1) / kTr));
+    k_transpose_g<<<tg, kBlock, 0, s>>>(grad_out, batch, n_post, Bp, gT, odd);
+    BS_CHECK_LAUNCH();
+#define BS_BT1(T, C, H, L)                                                                   \
+  k_matvec_vjp_bt<T, C, H, L><<<g, kBlock, 0, s>>>((const T*)spk, batch, n_pre, indptr, indices, \
+                                                   k, w, w_homo, n_post, grad_out, gT, Bp, odd, \
+                                                   (int32_t)(tg.x * tg.y), grad_spk, grad_w)
+#define BS_BT(T, C, H) do { if (lanes == 16) BS_BT1(T, C, H, 16); else BS_BT1(T, C, H, 64); } while (0)
+    if (spk_dtype == BS_SPK_U8) {
+      if (csr) { if (het) BS_BT(uint8_t, true, true); else BS_BT(uint8_t, true, false); }
+      else { if (het) BS_BT(uint8_t, false, true); else BS_BT(uint8_t, false, false); }
+    } else {
+      if (csr) { if (het) BS_BT(float, true, true); else BS_BT(float, true, false); }
+      else { if (het) BS_BT(float, false, true); else BS_BT(float, false, false); }
+    }
+#undef BS_BT
+#undef BS_BT1
+    BS_CHECK_LAUNCH();
+    return BS_OK;
+  }
+  // batch == 0 or n_post == 0 go through the kernel: it writes grad_w = 0 (g never read)
 #define BS_VJPB(T, C, H)                                                                    \
   k_matvec_vjp_batch<T, C, H><<<g, kBlock, 0, s>>>((const T*)spk, batch, n_pre, indptr,       \
                                                    indices, k, w, w_homo, n_post, grad_out,   \
@@ -863,6 +1072,37 @@ extern "C" int bs_event_matvec_vjp_batch_f32(const void* spk, int32_t spk_dtype,
 #undef BS_VJPB
   BS_CHECK_LAUNCH();
   return BS_OK;
+}
+
+}  // namespace
+
+extern "C" int bs_event_matvec_vjp_batch_f32(const void* spk, int32_t spk_dtype, int32_t batch,
+                                             int32_t n_pre, const int32_t* indptr,
+                                             const int32_t* indices, int32_t k, const float* w,
+                                             float w_homo, int32_t n_post, const float* grad_out,
+                                             float* grad_spk, float* grad_w,
+                                             bs_stream_t stream) {
+  bs_clear_error();
+  return vjp_batch(spk, spk_dtype, batch, n_pre, indptr, indices, k, w, w_homo, n_post, grad_out,
+                   grad_spk, grad_w, nullptr, 0, stream);
+}
+
+extern "C" size_t bs_event_matvec_vjp_batch_workspace_size(int32_t batch, int32_t n_pre,
+                                                           int32_t n_post) {
+  bs_clear_error();
+  return vjp_bt_bytes(batch, n_pre, n_post);
+}
+
+extern "C" int bs_event_matvec_vjp_batch_ws_f32(const void* spk, int32_t spk_dtype,
+                                                int32_t batch, int32_t n_pre,
+                                                const int32_t* indptr, const int32_t* indices,
+                                                int32_t k, const float* w, float w_homo,
+                                                int32_t n_post, const float* grad_out,
+                                                float* grad_spk, float* grad_w, void* workspace,
+                                                size_t workspace_bytes, bs_stream_t stream) {
+  bs_clear_error();
+  return vjp_batch(spk, spk_dtype, batch, n_pre, indptr, indices, k, w, w_homo, n_post, grad_out,
+                   grad_spk, grad_w, workspace, workspace_bytes, stream);
 }
 
 namespace {

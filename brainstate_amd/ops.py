@@ -184,10 +184,13 @@ def event_matvec_vjp_batch(spk, indices, w, n_post, grad_out, k=None, indptr=Non
     if need_w:
         gw = torch.empty((), dtype=torch.float32, device=dev) if homo else \
             torch.empty(w.shape, dtype=torch.float32, device=dev)
-    N.check(N.lib().bs_event_matvec_vjp_batch_f32(
+    nbytes = int(N.lib().bs_event_matvec_vjp_batch_workspace_size(B, n_pre, int(n_post)))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes > 0 else None
+    N.check(N.lib().bs_event_matvec_vjp_batch_ws_f32(
         N.ptr(spk), _spk_dtype(spk), B, n_pre, N.ptr(indptr), N.ptr(indices.contiguous()), k,
         None if homo else N.ptr(w.contiguous()), float(w) if homo else 0.0, int(n_post),
-        N.ptr(g), N.ptr(gs), N.ptr(gw), N.stream_handle(dev)), 'bs_event_matvec_vjp_batch_f32')
+        N.ptr(g), N.ptr(gs), N.ptr(gw), N.ptr(ws), nbytes, N.stream_handle(dev)),
+        'bs_event_matvec_vjp_batch_ws_f32')
     return gs, gw
 
 

@@ -137,6 +137,18 @@ BS_API int bs_event_matvec_vjp_batch_f32(const void* spk, int32_t spk_dtype, int
                                          float w_homo, int32_t n_post, const float* grad_out,
                                          float* grad_spk, float* grad_w, bs_stream_t stream);
 
+/* The same gradients with a workspace of bs_event_matvec_vjp_batch_workspace_size bytes, in
+ * which grad_out is held transposed (0: none is used).  grad_spk and per-synapse grad_w have
+ * the bits bs_event_matvec_vjp_batch_f32 gives. */
+BS_API size_t bs_event_matvec_vjp_batch_workspace_size(int32_t batch, int32_t n_pre,
+                                                       int32_t n_post);
+BS_API int bs_event_matvec_vjp_batch_ws_f32(const void* spk, int32_t spk_dtype, int32_t batch,
+                                            int32_t n_pre, const int32_t* indptr,
+                                            const int32_t* indices, int32_t k, const float* w,
+                                            float w_homo, int32_t n_post, const float* grad_out,
+                                            float* grad_spk, float* grad_w, void* workspace,
+                                            size_t workspace_bytes, bs_stream_t stream);
+
 /* ---------------------------------------------------------------- N2a, destination-bucketed
  * Same operator as bs_event_scatter_f32 / bs_event_matvec_f32 (replaces `EventArray(spk) @
  * FixedPostNumConn` / `@ CSR`, brainstate/nn/_event_fixedprob.py:176-181,192,202-205,249-252)

@@ -1,0 +1,55 @@
+"""GPU: gradients of a batch through the transposed form against the per-row kernel, bit for bit
+(grad_spk, and grad_w as the per-row gradients added in row order)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+# 16 and 64 batch lanes, one lane group past each, batches that end inside a group; rows of less
+# than one, one, and several chunks; tiles of the transposition cut on both sides
+@pytest.mark.parametrize('B,n_pre,n_post,k', [(3, 7000, 63, 65), (8, 50, 64, 64), (16, 300, 65, 17),
+                                              (17, 200, 1000, 80), (64, 129, 127, 128),
+                                              (65, 40, 1, 200), (130, 33, 500, 1), (9, 4, 4000, 1000)])
+@pytest.mark.parametrize('het', [True, False])
+@pytest.mark.parametrize('csr', [True, False])
+@pytest.mark.parametrize('odd', [True, False])
+def test_transposed_vjp_equals_rows(B, n_pre, n_post, k, het, csr, odd):
+    import torch
+    if not torch.cuda.is_available():
+        pytest.fail('GPU tests need a ROCm GPU')
+    from brainstate_amd import _native as N
+    from brainstate_amd import ops
+    print('[case] vjp batch', B, n_pre, n_post, k, het, csr, odd, flush=True)
+    assert N.lib().bs_event_matvec_vjp_batch_workspace_size(B, n_pre, n_post) > 0
+    rs = np.random.RandomState(B + k)
+    t = lambda a: torch.as_tensor(a, device='cuda')  # noqa: E731
+    idx = rs.randint(-2, n_post + 2, (n_pre, k)).astype(np.int32)
+    indptr = None
+    if csr:
+        lens = rs.randint(0, k + 1, n_pre)
+        indptr = t(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32))
+        idx = idx.reshape(-1)[:int(lens.sum())]
+    idx = t(idx)
+    w = t(rs.randn(*idx.shape).astype(np.float32)) if het else 0.7
+    x = t(np.where(rs.rand(B, n_pre) < 0.2, rs.rand(B, n_pre) + 0.1, 0).astype(np.float32))
+    g = rs.randn(B, n_post).astype(np.float32)
+    if odd:
+        g[B // 2, n_post // 2] = np.inf
+        g[0, 0] = np.nan
+    g = t(g)
+    gs, gw = ops.event_matvec_vjp_batch(x, idx, w, n_post, g, indptr=indptr)
+    same = lambda a, b: torch.equal(torch.nan_to_num(a, nan=7e30), torch.nan_to_num(b, nan=7e30))  # noqa: E731
+    total, absum = None, 0.0
+    for b in range(B):
+        a, c = ops.event_matvec_vjp(x[b], idx, w, n_post, g[b].contiguous(), indptr=indptr)
+        assert same(gs[b], a), b
+        total = c if total is None else total + c
+        absum += float(x[b].sum()) * k * float(g[b].abs().max())
+    if het:
+        assert same(gw, total)
+    elif not odd:
+        # n fp32 terms of one sum in another order: n 2^-24 of their absolute sum at most
+        assert abs(float(gw) - float(total)) <= 1e-5 * absum
+    only = ops.event_matvec_vjp_batch(x, idx, w, n_post, g, indptr=indptr, need_w=False)[0]
+    assert same(only, gs)
