@@ -125,6 +125,9 @@ SIGNATURES = {
     'bs_event_matvec_vjp_batch_f32': (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_vp, c_vp,
                                                      c_i32, c_vp, c_f32, c_i32, c_vp, c_vp,
                                                      c_vp, c_vp]),
+    'bs_matvec_workspace_size': (c_size, [c_i32, c_i32, c_i32, c_i32, c_i32]),
+    'bs_matvec_ws_f32': (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_vp, c_i32, c_vp,
+                                        c_f32, c_i32, c_vp, c_i32, c_vp, c_size, c_vp]),
     'bs_event_matvec_vjp_batch_workspace_size': (c_size, [c_i32, c_i32, c_i32]),
     'bs_event_matvec_vjp_batch_ws_f32': (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_vp, c_vp,
                                                         c_i32, c_vp, c_f32, c_i32, c_vp, c_vp,

@@ -11,6 +11,8 @@
 // the spike of each and adds the weight in column order, so every post accumulates its
 // incoming synapses in ascending (pre, k) order -- bit-identical to a sequential pre-major
 // scatter, with no atomics.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -271,6 +273,202 @@ __global__ __launch_bounds__(kBlock) void k_matvec(const T* __restrict__ spk, in
       if (v != 0.0f) bs_atomic_add_f32(out + j, v);
     }
   }
+}
+
+// The mat-vec (fixed fan-out) with the sums in LDS instead of global fp32 atomics, which run at
+// ~2e10/s over the whole chip.  Workgroup (range q, row group r) of batch row blockIdx.y lists
+// its active rows, reads all their synapses and adds those that hit its `len` posts; with one
+// row group it writes the outputs, else a partial row that k_mv_reduce adds (header, then
+// [R][n_post] per batch row).  As in the bucketed operator, the row groups in use follow the
+// spikes: every workgroup estimates the active synapses from the same leading rows, groups
+// past R_eff return, and R_eff = 1 writes the outputs.
+// A shared event weight is counted and added in one chain afterwards (the sequential sum, as
+// k_matvec and the bucketed operator give it); other sums are fp32 in no fixed order.
+// The workgroups of a row group read the same synapses: they are placed on one XCD.
+// Bound by the LDS fp32 adds (84 instead of 112 us with integer ones) and the re-reads of the
+// synapses by every range.
+constexpr int kMvB = 1024;
+constexpr int kMvPosts = 16000;        // posts per range at most (two workgroups per CU)
+constexpr int kMvSpan = 4096;          // rows listed at a time
+constexpr int kMvSample = 16384;       // leading rows the estimate reads
+constexpr int kMvSyn = 8192;           // active synapses per row group the estimate aims for,
+                                       // plus n_post / 4 (a group's partials cost that much)
+constexpr int kMvHdr = 64;             // header words ahead of a batch row's partials
+template <typename T, bool kHet, bool kVal>
+__global__ __launch_bounds__(kMvB) void k_mv_lds(
+    const T* __restrict__ spk, int32_t n_pre, const int32_t* __restrict__ indices, int32_t k,
+    const float* __restrict__ w, float w_homo, int32_t n_post, int32_t nr, int32_t len,
+    int32_t R, int32_t accumulate, float* __restrict__ out, uint32_t* __restrict__ ws) {
+  constexpr bool kCount = !kHet && !kVal;
+  constexpr int kWv = kMvB / BS_WAVE, kU = kMvSpan / kMvB;
+  __shared__ __align__(16) uint32_t s_acc[kMvPosts];
+  __shared__ int32_t s_list[kMvSpan];
+  __shared__ int32_t s_wave[kU][kWv];
+  const int lane = bs_lane();
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / BS_WAVE));
+  spk += (int64_t)blockIdx.y * n_pre;
+  out += (int64_t)blockIdx.y * n_post;
+  ws += (int64_t)blockIdx.y * (kMvHdr + (R > 1 ? (int64_t)R * n_post : 0));
+  // workgroup x -> (r, q): the ranges of a row group share x mod 8, the XCD
+  const int32_t x = blockIdx.x;
+  const int32_t r = R == 1 ? 0 : x / (8 * nr) * 8 + x % 8, q = R == 1 ? x : x / 8 % nr;
+  if (r >= R) return;
+  int32_t Reff = 1;
+  if (R > 1) {
+    const int32_t ns = n_pre < kMvSample ? n_pre : kMvSample;
+    int32_t c = 0;
+#pragma unroll
+    for (int u = 0; u < kMvSample / kMvB; ++u) {
+      const int32_t i = u * kMvB + threadIdx.x;
+      c += i < ns && spk[i < ns ? i : 0] != T(0) ? 1 : 0;
+    }
+#pragma unroll
+    for (int o = BS_WAVE / 2; o > 0; o >>= 1) c += __shfl_xor(c, o);
+    if (lane == 0) s_wave[0][wid] = c;
+    __syncthreads();
+    c = 0;
+#pragma unroll
+    for (int v = 0; v < kWv; ++v) c += s_wave[0][v];
+    __syncthreads();
+    const double syn = (double)c * (double)n_pre / (double)ns * (double)k;
+    // ... and no group lists more than one span of rows
+    const double re = ceil(syn / (kMvSyn + n_post / 4)), rs = ceil((double)n_pre / kMvSpan);
+    const double rw = re > rs ? re : rs;
+    Reff = rw > (double)R ? R : (int32_t)rw;
+    if (x == 0 && threadIdx.x == 0) ws[0] = (uint32_t)Reff;
+    if (r >= Reff) return;             // whole workgroup
+  }
+  const int32_t p0 = q * len;
+  const int32_t rest = n_post - p0 > 0 ? n_post - p0 : 0;     // 0: a last range left empty
+  const int32_t pn = rest < len ? rest : len;
+  for (int j = threadIdx.x; j < pn; j += kMvB) s_acc[j] = 0u;
+  const int64_t r0 = (int64_t)n_pre * r / Reff, r1 = (int64_t)n_pre * (r + 1) / Reff;
+  for (int64_t c0 = r0; c0 < r1; c0 += kMvSpan) {
+    uint64_t m[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int64_t i = c0 + u * kMvB + threadIdx.x;
+      m[u] = bs_ballot(i < r1 && spk[i < r1 ? i : r0] != T(0));
+      if (lane == 0) s_wave[u][wid] = __popcll(m[u]);
+    }
+    __syncthreads();                   // also: s_acc is zero, the last span's rows are done
+    int32_t count = 0;
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      int32_t pos = count;
+#pragma unroll
+      for (int v = 0; v < kWv; ++v) {
+        const int32_t n = s_wave[u][v];
+        pos += v < wid ? n : 0;
+        count += n;
+      }
+      if ((m[u] >> lane) & 1ull)
+        s_list[pos + bs_rank_below(m[u])] = (int32_t)(c0 + u * kMvB + threadIdx.x);
+    }
+    __syncthreads();
+    // eight 64-synapse chunks in flight per wave: two of each of four rows, or, when that would
+    // leave waves without rows, eight of one
+    auto rows = [&](auto nrow) {
+      constexpr int kRows = decltype(nrow)::value, kPass = 8 / kRows;
+      for (int32_t a0 = wid * kRows; a0 < count; a0 += kWv * kRows) {
+        int32_t row[kRows];
+        float xv[kRows];
+#pragma unroll
+        for (int e = 0; e < kRows; ++e) {
+          row[e] = __builtin_amdgcn_readfirstlane(s_list[a0 + e < count ? a0 + e : a0]);
+          xv[e] = kVal ? (float)spk[row[e]] : 1.0f;
+        }
+        for (int32_t t0 = 0; t0 < k; t0 += kPass * BS_WAVE) {
+          int32_t jj[kRows][kPass];
+          float vv[kRows][kPass];
+#pragma unroll
+          for (int e = 0; e < kRows; ++e)
+#pragma unroll
+            for (int u = 0; u < kPass; ++u) {
+              const int32_t t = t0 + u * BS_WAVE + lane;
+              const bool ok = t < k && a0 + e < count;
+              const int64_t o = (int64_t)row[e] * k + t;
+              jj[e][u] = ok ? indices[o] : -1;
+              vv[e][u] = kHet && ok ? w[o] : w_homo;
+            }
+#pragma unroll
+          for (int e = 0; e < kRows; ++e)
+#pragma unroll
+            for (int u = 0; u < kPass; ++u) {
+              const uint32_t j = (uint32_t)jj[e][u] - (uint32_t)p0;
+              if (jj[e][u] >= 0 && j < (uint32_t)pn) {
+                if (kCount) atomicAdd(&s_acc[j], 1u);
+                else unsafeAtomicAdd((float*)&s_acc[j], kVal ? vv[e][u] * xv[e] : vv[e][u]);
+              }
+            }
+        }
+      }
+    };
+    if (count <= 3 * kWv) rows(std::integral_constant<int, 1>());
+    else rows(std::integral_constant<int, 4>());
+    __syncthreads();                   // the list is rewritten next
+  }
+  __syncthreads();                     // a group without rows: s_acc is zero
+  if (Reff > 1) {
+    uint32_t* dst = ws + kMvHdr + (int64_t)r * n_post + p0;
+    for (int j = threadIdx.x; j < pn; j += kMvB) dst[j] = s_acc[j];
+    return;
+  }
+  for (int j = threadIdx.x; j < pn; j += kMvB) {
+    float acc = accumulate ? out[p0 + j] : 0.0f;
+    if (kCount) {
+      const uint32_t c = s_acc[j];
+      for (uint32_t u = 0; u < c; ++u) acc += w_homo;
+    } else {
+      acc += __uint_as_float(s_acc[j]);
+    }
+    out[p0 + j] = acc;
+  }
+}
+
+// out[j] = (accumulate ? out[j] : 0) + the R_eff partials of j.  A workgroup takes 64 posts;
+// thread (c, j) adds every fourth partial from c on, 16 in flight, and the four sums meet in
+// order.
+template <bool kCount>
+__global__ __launch_bounds__(kBlock) void k_mv_reduce(int32_t n_post, int32_t R, float w_homo,
+                                                      int32_t accumulate,
+                                                      const uint32_t* __restrict__ ws,
+                                                      float* __restrict__ out) {
+  constexpr int kC = kBlock / BS_WAVE, kF = 16;
+  __shared__ uint32_t s_p[kC][BS_WAVE];
+  const int c = threadIdx.x / BS_WAVE, lane = bs_lane();
+  const int64_t j = (int64_t)blockIdx.x * BS_WAVE + lane;
+  ws += (int64_t)blockIdx.y * (kMvHdr + (int64_t)R * n_post);
+  out += (int64_t)blockIdx.y * n_post;
+  const int32_t Reff = (int32_t)__builtin_amdgcn_readfirstlane(ws[0]);
+  if (Reff <= 1) return;
+  const uint32_t* p = ws + kMvHdr + (j < n_post ? j : 0);
+  float sum = 0.0f;
+  uint32_t cnt = 0;
+  for (int32_t g = c; g < Reff; g += kC * kF) {
+    uint32_t v[kF];
+#pragma unroll
+    for (int u = 0; u < kF; ++u)
+      v[u] = g + u * kC < Reff ? p[(int64_t)(g + u * kC) * n_post] : 0u;
+#pragma unroll
+    for (int u = 0; u < kF; ++u) {
+      if (kCount) cnt += v[u];
+      else sum += __uint_as_float(v[u]);
+    }
+  }
+  s_p[c][lane] = kCount ? cnt : __float_as_uint(sum);
+  __syncthreads();
+  if (c != 0 || j >= n_post) return;
+  float acc = accumulate ? out[j] : 0.0f;
+  if (kCount) {
+    cnt = s_p[0][lane] + s_p[1][lane] + s_p[2][lane] + s_p[3][lane];
+    for (uint32_t u = 0; u < cnt; ++u) acc += w_homo;
+  } else {
+    sum = __uint_as_float(s_p[0][lane]);
+    for (int u = 1; u < kC; ++u) sum += __uint_as_float(s_p[u][lane]);
+    acc += sum;
+  }
+  out[j] = acc;
 }
 
 // gw[0] += the sum over the workgroup's waves of their (wave-uniform) v: one atomic per
@@ -923,18 +1121,83 @@ extern "C" int bs_event_gather_f32(const uint32_t* spk_bits, int32_t n_pre,
 
 namespace {
 
+// Ranges and row groups of k_mv_lds; R = 0 where k_matvec is kept.  k_matvec costs ~12 us (with
+// the fill of its outputs) plus 5e-5 us per event, k_mv_lds ~20 us on a sparse layer and
+// 1e-5 us per event (us per call, k_matvec / k_mv_lds): 100k x 100k, K = 1000, p = 0.1 529 /
+// 125, 0.01 65 / 34, 0.002 19 / 23; one shared weight, 400k x 4k, K = 250, p = 0.2 870 / 119,
+// 0.002 23 / 19; 64 x 3200 -> 4000, K = 80, p = 0.05 43 / 17, 0.002 11 / 9; 128 x 10k, K = 100,
+// p = 0.2 1207 / 179.  The density is not known here: single vectors take it from 2e7
+// synapses (5e7 with a shared weight, whose calls are otherwise the shortest), batches of 8
+// (32) always; more than 8 ranges would read the synapses too often.
+struct MvPlan {
+  int32_t nr, len, R;
+};
+
+MvPlan mv_plan(int32_t batch, int32_t n_pre, int32_t k, int32_t n_post, bool csr, bool count) {
+  MvPlan p{0, 0, 0};
+  if (csr || batch < 1 || n_pre < 1 || n_post < 1 || k < 1) return p;
+  const int32_t least = (n_post + kMvPosts - 1) / kMvPosts;
+  if (least > 8) return p;
+  const double syn = (double)n_pre * k;
+  if (batch < (count ? 32 : 8) && syn * batch < (count ? 5e7 : 2e7)) return p;
+  int32_t nr = least, R = 1;
+  if (batch >= 8) {
+    const int32_t want = 512 / batch < 8 ? 512 / batch : 8;
+    const int32_t most = (n_post + 255) / 256;
+    nr = want > nr ? want : nr;
+    nr = nr < most ? nr : (most > least ? most : least);
+  }
+  const int64_t wgs = (int64_t)batch * nr;
+  if (wgs < 256) {
+    const int64_t rows = ((int64_t)n_pre + 63) / 64;
+    const int64_t g = 512 / wgs;
+    R = (int32_t)(g < rows ? g : rows);
+    if (R < 1) R = 1;
+  }
+  return MvPlan{nr, (n_post + nr - 1) / nr, R};
+}
+
+size_t mv_ws_bytes(const MvPlan& p, int32_t batch, int32_t n_post) {
+  return p.R > 1 ? (size_t)batch * (kMvHdr + (size_t)p.R * n_post) * 4 : 0;
+}
+
 // Shared launcher of the fused mat-vec (event or value-weighted).
 template <bool kVal>
 int matvec_launch(const void* spk, int32_t spk_dtype, int32_t batch, int32_t n_pre,
                   const int32_t* indptr, const int32_t* indices, int32_t k, const float* w,
-                  float w_homo, int32_t n_post, float* out, int32_t accumulate, hipStream_t s,
-                  const char* who) {
+                  float w_homo, int32_t n_post, float* out, int32_t accumulate, void* ws,
+                  size_t ws_bytes, hipStream_t s, const char* who) {
   BS_CHECK_ARG(n_pre >= 0 && n_post >= 0, "%s: negative size", who);
   BS_CHECK_ARG(batch >= 1 && batch <= 65535, "%s: batch %d outside [1, 65535]", who, batch);
   BS_CHECK_ARG(indptr != nullptr || k >= 0, "%s: k=%d < 0", who, k);
   BS_CHECK_ARG(spk_dtype == BS_SPK_U8 || spk_dtype == BS_SPK_F32, "%s: unknown spike dtype %d",
                who, spk_dtype);
   if (n_post > 0) BS_CHECK_ARG(out != nullptr, "%s: out is NULL", who);
+  const MvPlan mp = mv_plan(batch, n_pre, k, n_post, indptr != nullptr, !kVal && w == nullptr);
+  const size_t mneed = mv_ws_bytes(mp, batch, n_post);
+  if (mp.R > 0 && (mneed == 0 || ws != nullptr)) {
+    BS_CHECK_ARG(spk && indices, "%s: NULL pointer", who);
+    BS_CHECK_ARG(ws_bytes >= mneed, "%s: workspace of %zu bytes needed (got %zu)", who, mneed,
+                 ws_bytes);
+    const dim3 mg((unsigned)(mp.R == 1 ? mp.nr : (mp.R + 7) / 8 * 8 * mp.nr), (unsigned)batch);
+    const dim3 rg((unsigned)(((int64_t)n_post + BS_WAVE - 1) / BS_WAVE), (unsigned)batch);
+    uint32_t* part = (uint32_t*)ws;
+#define BS_ML(T, H)                                                                        \
+  k_mv_lds<T, H, kVal><<<mg, kMvB, 0, s>>>((const T*)spk, n_pre, indices, k, w, w_homo, n_post, \
+                                           mp.nr, mp.len, mp.R, accumulate, out, part)
+    if (spk_dtype == BS_SPK_U8) { if (w) BS_ML(uint8_t, true); else BS_ML(uint8_t, false); }
+    else { if (w) BS_ML(float, true); else BS_ML(float, false); }
+#undef BS_ML
+    BS_CHECK_LAUNCH();
+    if (mp.R > 1) {
+      if (w || kVal)
+        k_mv_reduce<false><<<rg, kBlock, 0, s>>>(n_post, mp.R, w_homo, accumulate, part, out);
+      else
+        k_mv_reduce<true><<<rg, kBlock, 0, s>>>(n_post, mp.R, w_homo, accumulate, part, out);
+      BS_CHECK_LAUNCH();
+    }
+    return BS_OK;
+  }
   if (!accumulate) {
     int rc = bs_fill_f32(out, (int64_t)batch * n_post, 0.0f, s);
     if (rc) return rc;
@@ -973,7 +1236,7 @@ extern "C" int bs_event_matvec_f32(const void* spk, int32_t spk_dtype, int32_t n
                                    int32_t accumulate, bs_stream_t stream) {
   bs_clear_error();
   return matvec_launch<false>(spk, spk_dtype, 1, n_pre, indptr, indices, k, w, w_homo, n_post,
-                              out, accumulate, bs_stream(stream), "bs_event_matvec_f32");
+                              out, accumulate, nullptr, 0, bs_stream(stream), "bs_event_matvec_f32");
 }
 
 extern "C" int bs_event_matvec_batch_f32(const void* spk, int32_t spk_dtype, int32_t batch,
@@ -983,7 +1246,7 @@ extern "C" int bs_event_matvec_batch_f32(const void* spk, int32_t spk_dtype, int
                                          int32_t accumulate, bs_stream_t stream) {
   bs_clear_error();
   return matvec_launch<false>(spk, spk_dtype, batch, n_pre, indptr, indices, k, w, w_homo,
-                              n_post, out, accumulate, bs_stream(stream),
+                              n_post, out, accumulate, nullptr, 0, bs_stream(stream),
                               "bs_event_matvec_batch_f32");
 }
 
@@ -993,7 +1256,7 @@ extern "C" int bs_value_matvec_f32(const float* x, int32_t n_pre, const int32_t*
                                    bs_stream_t stream) {
   bs_clear_error();
   return matvec_launch<true>(x, BS_SPK_F32, 1, n_pre, indptr, indices, k, w, w_homo, n_post,
-                             out, accumulate, bs_stream(stream), "bs_value_matvec_f32");
+                             out, accumulate, nullptr, 0, bs_stream(stream), "bs_value_matvec_f32");
 }
 
 extern "C" int bs_value_matvec_batch_f32(const float* x, int32_t batch, int32_t n_pre,
@@ -1002,7 +1265,28 @@ extern "C" int bs_value_matvec_batch_f32(const float* x, int32_t batch, int32_t 
                                          float* out, int32_t accumulate, bs_stream_t stream) {
   bs_clear_error();
   return matvec_launch<true>(x, BS_SPK_F32, batch, n_pre, indptr, indices, k, w, w_homo, n_post,
-                             out, accumulate, bs_stream(stream), "bs_value_matvec_batch_f32");
+                             out, accumulate, nullptr, 0, bs_stream(stream),
+                             "bs_value_matvec_batch_f32");
+}
+
+extern "C" size_t bs_matvec_workspace_size(int32_t batch, int32_t n_pre, int32_t k,
+                                           int32_t n_post, int32_t count) {
+  bs_clear_error();
+  return mv_ws_bytes(mv_plan(batch, n_pre, k, n_post, false, count != 0), batch, n_post);
+}
+
+extern "C" int bs_matvec_ws_f32(const void* spk, int32_t spk_dtype, int32_t value, int32_t batch,
+                                int32_t n_pre, const int32_t* indices, int32_t k, const float* w,
+                                float w_homo, int32_t n_post, float* out, int32_t accumulate,
+                                void* workspace, size_t workspace_bytes, bs_stream_t stream) {
+  bs_clear_error();
+  hipStream_t s = bs_stream(stream);
+  return value ? matvec_launch<true>(spk, spk_dtype, batch, n_pre, nullptr, indices, k, w, w_homo,
+                                     n_post, out, accumulate, workspace, workspace_bytes, s,
+                                     "bs_matvec_ws_f32")
+               : matvec_launch<false>(spk, spk_dtype, batch, n_pre, nullptr, indices, k, w,
+                                      w_homo, n_post, out, accumulate, workspace,
+                                      workspace_bytes, s, "bs_matvec_ws_f32");
 }
 
 namespace {

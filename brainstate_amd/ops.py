@@ -80,21 +80,52 @@ def _batch_of(x):
     return lead, math.prod(lead), int(x.shape[-1]) if x.dim() else 1
 
 
+def _fixed_matvec(x, value, indices, k, w, n_post, out, accumulate, batch, n_pre):
+    """bs_matvec_ws_f32 of the rows of ``x`` [batch, n_pre] (contiguous) onto ``out``; its
+    workspace is kept per (device, stream)."""
+    dev = indices.device
+    homo = not torch.is_tensor(w) or w.numel() == 1
+    idx = indices.contiguous()
+    wt = None if homo else w.contiguous()
+    raw = N.raw_stream(dev)
+    lib = N.lib()
+    for b0 in range(0, batch, 65535):
+        nb = min(65535, batch - b0)
+        nbytes = int(lib.bs_matvec_workspace_size(nb, n_pre, k, n_post,
+                                                  1 if homo and not value else 0))
+        ws = None
+        if nbytes > 0:
+            ws = _WS_CACHE.get(('matvec', dev.index, raw))
+            if ws is None or ws.numel() < nbytes:
+                ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+                _WS_CACHE[('matvec', dev.index, raw)] = ws
+        xs, ys = (x, out) if nb == batch else (x.reshape(batch, n_pre)[b0:b0 + nb],
+                                               out.reshape(batch, n_post)[b0:b0 + nb])
+        N.check(lib.bs_matvec_ws_f32(
+            N.ptr(xs), _spk_dtype(x), 1 if value else 0, nb, n_pre, N.ptr(idx), k, N.ptr(wt),
+            float(w) if homo else 0.0, n_post, N.ptr(ys), 1 if accumulate else 0, N.ptr(ws),
+            nbytes, ctypes.c_void_p(raw)), 'bs_matvec_ws_f32')
+    return out
+
+
 def event_matvec(spk, indices, w, n_post, k=None, indptr=None, out=None, accumulate=False):
-    """Event mat-vec straight from the spike vector (one fused compaction + scatter launch);
-    ``spk`` [..., n_pre] with leading batch dimensions gives [..., n_post] in one launch."""
+    """Event mat-vec straight from the spike vector (one fused compaction + scatter launch, or
+    sums in LDS on large layers); ``spk`` [..., n_pre] with leading batch dimensions gives
+    [..., n_post] in one launch."""
     spk = _spk_view(spk)
     dev = indices.device
     lead, batch, n_pre = _batch_of(spk)
     k = _rows(n_pre, indices, k, indptr)
-    homo = not torch.is_tensor(w) or w.numel() == 1
-    w_homo = float(w) if homo else 0.0
     if out is None:
         out = torch.empty(lead + (n_post,), dtype=torch.float32, device=dev)
         accumulate = False
+    if indptr is None:
+        return _fixed_matvec(spk, False, indices, k, w, int(n_post), out, accumulate, batch,
+                             n_pre)
+    homo = not torch.is_tensor(w) or w.numel() == 1
     args = (N.ptr(indptr), N.ptr(indices.contiguous()), k,
-            None if homo else N.ptr(w.contiguous()), w_homo, int(n_post), N.ptr(out),
-            1 if accumulate else 0, N.stream_handle(dev))
+            None if homo else N.ptr(w.contiguous()), float(w) if homo else 0.0, int(n_post),
+            N.ptr(out), 1 if accumulate else 0, N.stream_handle(dev))
     if spk.dim() <= 1:
         N.check(N.lib().bs_event_matvec_f32(N.ptr(spk), _spk_dtype(spk), n_pre, *args),
                 'bs_event_matvec_f32')
@@ -126,10 +157,12 @@ def value_matvec(x, indices, w, n_post, k=None, indptr=None, out=None, accumulat
     dev = indices.device
     lead, batch, n_pre = _batch_of(x)
     k = _rows(n_pre, indices, k, indptr)
-    homo = not torch.is_tensor(w) or w.numel() == 1
     if out is None:
         out = torch.empty(lead + (n_post,), dtype=torch.float32, device=dev)
         accumulate = False
+    if indptr is None:
+        return _fixed_matvec(x, True, indices, k, w, int(n_post), out, accumulate, batch, n_pre)
+    homo = not torch.is_tensor(w) or w.numel() == 1
     wp, wh = (None, float(w)) if homo else (N.ptr(w.contiguous()), 0.0)
     if x.dim() <= 1:
         N.check(N.lib().bs_value_matvec_f32(

@@ -137,6 +137,17 @@ BS_API int bs_event_matvec_vjp_batch_f32(const void* spk, int32_t spk_dtype, int
                                          float w_homo, int32_t n_post, const float* grad_out,
                                          float* grad_spk, float* grad_w, bs_stream_t stream);
 
+/* bs_event_matvec_batch_f32 (value = 0) or bs_value_matvec_batch_f32 (value = 1) of a fixed
+ * fan-out connectivity with a workspace of bs_matvec_workspace_size bytes (0: none is used;
+ * count = 1 for events of one shared weight, else 0), in which large layers keep partial sums
+ * instead of adding to `out` atomically. */
+BS_API size_t bs_matvec_workspace_size(int32_t batch, int32_t n_pre, int32_t k, int32_t n_post,
+                                       int32_t count);
+BS_API int bs_matvec_ws_f32(const void* spk, int32_t spk_dtype, int32_t value, int32_t batch,
+                            int32_t n_pre, const int32_t* indices, int32_t k, const float* w,
+                            float w_homo, int32_t n_post, float* out, int32_t accumulate,
+                            void* workspace, size_t workspace_bytes, bs_stream_t stream);
+
 /* The same gradients with a workspace of bs_event_matvec_vjp_batch_workspace_size bytes, in
  * which grad_out is held transposed (0: none is used).  grad_spk and per-synapse grad_w have
  * the bits bs_event_matvec_vjp_batch_f32 gives. */
