@@ -101,3 +101,5 @@ __device__ __forceinline__ uint64_t* bs_scan_status(bs_scan_ws* ws) {
   return (uint64_t*)((char*)ws + BS_SCAN_WS_HEADER);
 }
 int bs_fill_f32(float* p, int64_t n, float v, hipStream_t s);
+int bs_max_indegree(int64_t n, int32_t n_pre, const int32_t* indptr, const int32_t* indices,
+                    int32_t n_post, uint32_t* deg, hipStream_t s);

@@ -818,20 +818,16 @@ __global__ __launch_bounds__(kBlock) void k_offsets(int nb, const uint32_t* cap,
   }
 }
 
-// Per-synapse weights: in-degree of every neuron per kind (valid targets) and the bit
-// pattern of max |w| per kind (all weights of the kind).
-__global__ __launch_bounds__(256) void k_indeg(NetArgs a, uint32_t* deg, WsHeader* hdr) {
+// Per-synapse weights: the bit pattern of max |w| per kind (all weights of the kind).
+__global__ __launch_bounds__(256) void k_wbits(NetArgs a, WsHeader* hdr) {
   const int64_t tot_e = (int64_t)a.n_exc * a.k_e;
   const int64_t tot = tot_e + (int64_t)(a.n - a.n_exc) * a.k_i;
   uint32_t wb[2] = {0u, 0u};
   for (int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; s < tot;
        s += (int64_t)gridDim.x * blockDim.x) {
     const int k = s >= tot_e ? 1 : 0;
-    const int64_t o = k ? s - tot_e : s;
-    const int32_t tgt = k ? a.idx_i[o] : a.idx_e[o];
-    const uint32_t b = __float_as_uint(k ? a.w_i[o] : a.w_e[o]) & 0x7FFFFFFFu;
+    const uint32_t b = __float_as_uint(k ? a.w_i[s - tot_e] : a.w_e[s]) & 0x7FFFFFFFu;
     wb[k] = b > wb[k] ? b : wb[k];
-    if ((uint32_t)tgt < (uint32_t)a.n) atomicAdd(&deg[(int64_t)k * a.n + tgt], 1u);
   }
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
@@ -846,39 +842,22 @@ __global__ __launch_bounds__(256) void k_indeg(NetArgs a, uint32_t* deg, WsHeade
 
 // S per kind from D = max in-degree and W = max |w|: with W < 2^e_w and D <= 2^e_d,
 // S = 30 - e_w - e_d (at most 100) keeps |sum of rounded weights| < 2^30 + D/2 < 2^31.
-// A weight that is not finite, or S < -100, sets error 2.  One workgroup.
-__global__ __launch_bounds__(kBlock) void k_qexp(int32_t n, const uint32_t* deg, WsHeader* hdr) {
-  __shared__ uint32_t s_max[2][kWaves];
-  uint32_t m[2] = {0u, 0u};
-  for (int64_t j = threadIdx.x; j < n; j += kBlock) {
-    const uint32_t de = deg[j], di = deg[(int64_t)n + j];
-    m[0] = de > m[0] ? de : m[0];
-    m[1] = di > m[1] ? di : m[1];
-  }
-#pragma unroll
+// A weight that is not finite, or S < -100, sets error 2.  D is deg[0] and deg[n] (the largest
+// in-degree of each kind).
+__global__ void k_qexp(int32_t n, const uint32_t* deg, WsHeader* hdr) {
+  if (threadIdx.x != 0) return;
   for (int k = 0; k < 2; ++k) {
-    for (int o = BS_WAVE / 2; o > 0; o >>= 1) {
-      const uint32_t v = __shfl_xor(m[k], o);
-      m[k] = v > m[k] ? v : m[k];
+    const uint32_t D = deg[(int64_t)k * n];
+    const uint32_t wb = hdr->wbits[k];
+    const int e_w = (wb >> 23) ? (int)(wb >> 23) - 126 : -126;
+    const int e_d = D <= 1 ? 0 : 32 - __clz(D - 1);
+    int S = 30 - e_w - e_d;
+    if (S > 100) S = 100;
+    if (wb >= 0x7F800000u || S < -100) {
+      hdr->error = 2u;
+      S = 0;
     }
-    if (bs_lane() == 0) s_max[k][threadIdx.x / BS_WAVE] = m[k];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 0; k < 2; ++k) {
-      uint32_t D = 0;
-      for (int w = 0; w < kWaves; ++w) D = s_max[k][w] > D ? s_max[k][w] : D;
-      const uint32_t wb = hdr->wbits[k];
-      const int e_w = (wb >> 23) ? (int)(wb >> 23) - 126 : -126;
-      const int e_d = D <= 1 ? 0 : 32 - __clz(D - 1);
-      int S = 30 - e_w - e_d;
-      if (S > 100) S = 100;
-      if (wb >= 0x7F800000u || S < -100) {
-        hdr->error = 2u;
-        S = 0;
-      }
-      hdr->qexp[k] = S;
-    }
+    hdr->qexp[k] = S;
   }
 }
 
@@ -1138,9 +1117,14 @@ extern "C" int bs_net_prepare(const bs_net* net, void* workspace, bs_stream_t st
   BS_CHECK_LAUNCH();
   if (net->w_e) {  // fixed-point exponents of the per-synapse weights
     uint32_t* deg = (uint32_t*)(ws + L.off_deg);
-    k_indeg<<<2048, 256, 0, s>>>(a, deg, (WsHeader*)ws);
+    k_wbits<<<2048, 256, 0, s>>>(a, (WsHeader*)ws);
     BS_CHECK_LAUNCH();
-    k_qexp<<<1, kBlock, 0, s>>>(net->n, deg, (WsHeader*)ws);
+    rc = bs_max_indegree((int64_t)a.n_exc * a.k_e, 0, nullptr, a.idx_e, net->n, deg, s);
+    if (rc) return rc;
+    rc = bs_max_indegree((int64_t)(a.n - a.n_exc) * a.k_i, 0, nullptr, a.idx_i, net->n,
+                         deg + net->n, s);
+    if (rc) return rc;
+    k_qexp<<<1, BS_WAVE, 0, s>>>(net->n, deg, (WsHeader*)ws);
     BS_CHECK_LAUNCH();
   }
   k_caps<<<L.nb, kBlock, 0, s>>>(a, (uint32_t*)(ws + L.off_cap));

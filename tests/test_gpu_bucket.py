@@ -454,3 +454,27 @@ def test_bucket_batch_equals_rows(torch_cuda, B, n_pre, n_post, k, p, het, sdt):
     assert torch.equal(ops.event_bucket_batch(wide, L), out)
     with pytest.raises(ValueError):
         ops.event_bucket_batch(x[:, :-1], L)
+
+
+# the in-degrees behind the exponent, counted in LDS: ranges of 40,000 posts met exactly, one
+# over, one post, and an index array that is not 16-byte aligned
+@pytest.mark.parametrize('n_post', [1, 40_000, 40_001, 123_457])
+@pytest.mark.parametrize('shift', [0, 1])
+def test_bucket_exponent_of_large_layouts(torch_cuda, n_post, shift):
+    torch = torch_cuda
+    from brainstate_amd import ops
+    say('bucket exponent', n_post, shift)
+    n_pre, k = 50_003, 81
+    gen = torch.Generator(device='cuda').manual_seed(n_post)
+    flat = torch.randint(-3, n_post + 3, (n_pre * k + 1,), device='cuda', generator=gen,
+                         dtype=torch.int32)
+    flat[::5] = 0                                   # a hub
+    idx = flat[shift:shift + n_pre * k].reshape(n_pre, k)
+    w = torch.full((n_pre, k), 0.6, device='cuda')
+    L = ops.build_buckets(idx, n_post, w=w)
+    v = idx.reshape(-1)
+    v = v[(v >= 0) & (v < n_post)].long()
+    D = int(torch.bincount(v, minlength=n_post).max())
+    e_d = int(np.ceil(np.log2(D))) if D > 1 else 0   # D <= 2^e_d
+    assert 2 ** e_d >= D > 2 ** (e_d - 1)
+    assert int(L['qexp']) == min(30 - 0 - e_d, 100)  # 0.6 < 2^0
