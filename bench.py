@@ -456,7 +456,7 @@ def bench_compact(args):
 def bench_vjp(args):
     """Reverse mode of the two event products (row f2): the event mat-vec at configs[1]'s shape
     (100k x 100k, K = 1000, per-synapse w, spikes at p = 0.1, a dense upstream gradient):
-    grad_spk and grad_w by k_matvec_vjp, one wave per pre row gathering g[idx]; and EventLinear
+    grad_spk and grad_w by k_matvec_vjp_lds, ranges of g passing through LDS; and EventLinear
     at configs[3]'s shape (spikes [64, 4096] at 5 %, W [4096, 4096]): grad_spk = g W^T by
     k_dense_gx and grad_W = spk^T g by k_dense_gw.  Byte models: mat-vec n_pre K (4 + 4 + 4)
     (indices and weights read, grad_w written; g gathered from L2) + n_pre (1 + 4) + n_post 4;

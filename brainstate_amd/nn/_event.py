@@ -3,9 +3,9 @@
 * ``FixedNumConn`` / ``EventFixedNumConn`` / ``EventFixedProb`` --
   brainstate/nn/_event_fixedprob.py:65-255.  Same arguments, validation and connectivity
   stream (numpy MT19937 ``randint`` with replacement, :161-171); ``update(spk)`` runs the
-  fused HIP spike-vector event mat-vec (C ABI ``bs_event_matvec_f32``: per-workgroup
-  compaction of the spike vector, then the pre-major scatter of the active rows) instead of
-  brainevent's kernel.
+  fused HIP spike-vector event mat-vec (C ABI ``bs_matvec_ws_f32``: per-workgroup compaction
+  of the spike vector, then the pre-major scatter of the active rows, or sums in LDS on large
+  layers and batches) instead of brainevent's kernel.
   With ``event_kernel='bucket'`` (or ``'auto'`` with per-synapse weights, or with a
   homogeneous weight onto more than 16,384 neurons whose rows average at least 4 synapses
   per destination bucket), the event path of inference runs the
