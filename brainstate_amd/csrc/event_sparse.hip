@@ -472,18 +472,19 @@ __global__ __launch_bounds__(kBlock) void k_mv_reduce(int32_t n_post, int32_t R,
 }
 
 // gw[0] += the sum over the workgroup's waves of their (wave-uniform) v: one atomic per
-// workgroup.  Called by every wave that has not ended.  (One per active row made the shared
+// workgroup.  The terms of this one sum mostly cancel, so it is carried in 64 bits up to the
+// atomic.  Called by every wave that has not ended.  (One per active row made the shared
 // weight's gradient of 100k rows of 128 synapses take 1.27 ms.)
 template <int kWaves>
-__device__ __forceinline__ void block_atomic_sum(float v, float* gw) {
-  __shared__ float s_v[kWaves];
+__device__ __forceinline__ void block_atomic_sum(double v, float* gw) {
+  __shared__ double s_v[kWaves];
   const int wid = threadIdx.x / BS_WAVE;
   if (bs_lane() == 0) s_v[wid] = v;
   __syncthreads();
   if (threadIdx.x != 0) return;
-  float t = s_v[0];
+  double t = s_v[0];
   for (int u = 1; u < kWaves; ++u) t += s_v[u];
-  if (t != 0.0f) bs_atomic_add_f32(gw, t);
+  if (t != 0.0) bs_atomic_add_f32(gw, (float)t);
 }
 
 constexpr int kVjpU = 8;  // 64-synapse chunks per wave and round in k_matvec_vjp
@@ -506,7 +507,7 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp(const T* __restrict__ spk
   const int lane = bs_lane();
   const int64_t nw = (int64_t)gridDim.x * (kBlock / BS_WAVE);
   const int32_t nnz = kCsr ? indptr[n_pre] : 0;
-  float sw = 0.0f;
+  double sw = 0.0;
   for (int64_t row = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / BS_WAVE; row < n_pre;
        row += nw) {
     int64_t beg, end;
@@ -552,7 +553,7 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp(const T* __restrict__ spk
       sg += __shfl_xor(sg, o);
     }
     if (lane == 0 && gx) gx[row] = sx;
-    if (!kHet && xv != 0.0f) sw += xv * sg;
+    if (!kHet && xv != 0.0f) sw += (double)xv * (double)sg;
   }
   if (!kHet && gw) block_atomic_sum<kBlock / BS_WAVE>(sw, gw);
 }
@@ -672,7 +673,7 @@ __global__ __launch_bounds__(kLvB) void k_matvec_vjp_lds(
         ahead(t + 2);
         __syncthreads();
       }
-      if (!kHet && gw) block_atomic_sum<kLvB / BS_WAVE>(0.0f, gw);
+      if (!kHet && gw) block_atomic_sum<kLvB / BS_WAVE>(0.0, gw);
       return;
     }
   }
@@ -702,7 +703,8 @@ __global__ __launch_bounds__(kLvB) void k_matvec_vjp_lds(
     for (int s = 0; s < kLvS; ++s) jj[s] = rd(indices + rowat(r + s / CP), syn(b, s % CP, ln));
   };
   load_idx(0, 0);
-  float cx[kR], cg[kR], sw = 0.0f;                    // lane sums carried over a row's blocks
+  float cx[kR], cg[kR];                               // lane sums carried over a row's blocks
+  double sw = 0.0;
   int32_t row = 0, kb = 0;                            // this pass: rows row .. row + kR - 1
   int step = 0;
   for (int32_t pass = 0; pass < passes; ++pass) {
@@ -758,7 +760,7 @@ __global__ __launch_bounds__(kLvB) void k_matvec_vjp_lds(
         const bool own = row + r < rows;
         const float vx = wave_sum_xor(sx);
         if (gx && own && lane == 0) gx[r0 + row + r] = vx;
-        if (!kHet && own && xv != 0.0f) sw += xv * wave_sum_xor(sg);
+        if (!kHet && own && xv != 0.0f) sw += (double)xv * (double)wave_sum_xor(sg);
       }
     }
     row = nrow;
@@ -886,7 +888,7 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp_bt(
   if (kHet && gw)
     for (int32_t t = lane; t < n_odd; t += BS_WAVE) all |= odd[t] != 0u;
   all = bs_ballot(all) != 0ull;
-  float sw = 0.0f;
+  double sw = 0.0;
   for (int64_t row = __builtin_amdgcn_readfirstlane(
            (int)(((int64_t)blockIdx.x * kBlock + threadIdx.x) / BS_WAVE));
        row < n_pre; row += nw) {
@@ -904,7 +906,8 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp_bt(
       for (int32_t b0 = 0; b0 < batch; b0 += LB) {
         const int32_t b = b0 + bl;
         const float* gb = gT + b;                      // b < Bp
-        float acc[A], tot = 0.0f;
+        float acc[A];
+        double tot = 0.0;
 #pragma unroll
         for (int a = 0; a < A; ++a) acc[a] = 0.0f;
         for (int64_t s0 = beg; s0 < end; s0 += BS_WAVE) {
@@ -930,7 +933,7 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp_bt(
                                             __float_as_uint(wl), l))
                                       : __shfl(wl, l + q);
               acc[a0 + u] += ws * v[u];
-              if (!kHet) tot += v[u];
+              if (!kHet) tot += (double)v[u];
             }
           }
         }
@@ -945,7 +948,7 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp_bt(
           if (gx && q == 0) gx[(int64_t)b * n_pre + row] = sx;
           if (!kHet && gw) {
             const float xv = (float)spk[(int64_t)b * n_pre + row];
-            if (xv != 0.0f) sw += xv * tot;            // this lane's share of the row's g
+            if (xv != 0.0f) sw += (double)xv * tot;    // this lane's share of the row's g
           }
         }
       }
