@@ -80,9 +80,16 @@ def _batch_of(x):
     return lead, math.prod(lead), int(x.shape[-1]) if x.dim() else 1
 
 
+def _call_workspace(nbytes, device):
+    """Uninitialised workspace of one call (None for 0 bytes), returned to torch's allocator
+    behind the call's kernels.  Not kept per stream: a captured graph would go on using it
+    after a larger call had replaced it, and two threads on one stream would share it between
+    the launches of one call."""
+    return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes > 0 else None
+
+
 def _fixed_matvec(x, value, indices, k, w, n_post, out, accumulate, batch, n_pre):
-    """bs_matvec_ws_f32 of the rows of ``x`` [batch, n_pre] (contiguous) onto ``out``; its
-    workspace is kept per (device, stream)."""
+    """bs_matvec_ws_f32 of the rows of ``x`` [batch, n_pre] (contiguous) onto ``out``."""
     dev = indices.device
     homo = not torch.is_tensor(w) or w.numel() == 1
     idx = indices.contiguous()
@@ -93,12 +100,7 @@ def _fixed_matvec(x, value, indices, k, w, n_post, out, accumulate, batch, n_pre
         nb = min(65535, batch - b0)
         nbytes = int(lib.bs_matvec_workspace_size(nb, n_pre, k, n_post,
                                                   1 if homo and not value else 0))
-        ws = None
-        if nbytes > 0:
-            ws = _WS_CACHE.get(('matvec', dev.index, raw))
-            if ws is None or ws.numel() < nbytes:
-                ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-                _WS_CACHE[('matvec', dev.index, raw)] = ws
+        ws = _call_workspace(nbytes, dev)
         xs, ys = (x, out) if nb == batch else (x.reshape(batch, n_pre)[b0:b0 + nb],
                                                out.reshape(batch, n_post)[b0:b0 + nb])
         N.check(lib.bs_matvec_ws_f32(
@@ -218,7 +220,7 @@ def event_matvec_vjp_batch(spk, indices, w, n_post, grad_out, k=None, indptr=Non
         gw = torch.empty((), dtype=torch.float32, device=dev) if homo else \
             torch.empty(w.shape, dtype=torch.float32, device=dev)
     nbytes = int(N.lib().bs_event_matvec_vjp_batch_workspace_size(B, n_pre, int(n_post)))
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes > 0 else None
+    ws = _call_workspace(nbytes, dev)
     N.check(N.lib().bs_event_matvec_vjp_batch_ws_f32(
         N.ptr(spk), _spk_dtype(spk), B, n_pre, N.ptr(indptr), N.ptr(indices.contiguous()), k,
         None if homo else N.ptr(w.contiguous()), float(w) if homo else 0.0, int(n_post),
@@ -462,19 +464,15 @@ def event_bucket_batch(spk, layout, out=None, accumulate=False):
     if out is None:
         out = torch.empty((B, L['n_post']), dtype=torch.float32, device=dev)
     sh = N.raw_stream(dev)
-    key = ('bucket', dev.index, sh)
     for b0 in range(0, B, 65535):
         nb = min(65535, B - b0)
         nbytes = int(N.lib().bs_event_bucket_batch_workspace_size(nb, n_pre, L['n_post'],
                                                                   L['nb']))
-        ws = _WS_CACHE.get(key)
-        if nbytes > 0 and (ws is None or ws.numel() < nbytes):
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-            _WS_CACHE[key] = ws
+        ws = _call_workspace(nbytes, dev)
         N.check(N.lib().bs_event_bucket_batch_f32(
             N.ptr(spk[b0:b0 + nb]), _spk_dtype(spk), nb, *fixed, N.ptr(out[b0:b0 + nb]),
-            1 if accumulate else 0, N.ptr(ws) if nbytes > 0 else None, nbytes,
-            ctypes.c_void_p(sh)), 'bs_event_bucket_batch_f32')
+            1 if accumulate else 0, N.ptr(ws), nbytes, ctypes.c_void_p(sh)),
+            'bs_event_bucket_batch_f32')
     return out
 
 
