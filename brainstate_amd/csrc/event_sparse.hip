@@ -834,33 +834,42 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp_batch(
 // ---- the same with g transposed: gT[j][b], Bp columns (a multiple of LB), row n_post zero ----
 // A 4-byte gather of g moves a line for each (synapse, batch row); transposed, the batch values
 // of a synapse's target lie side by side.
-constexpr int kTr = 64;   // tile of the transposition
+constexpr int kTr = 64;        // tile of the transposition
+constexpr int kTrWgs = 2048;   // its workgroups at most, a flag each: k_matvec_vjp_bt reads them all
+// Tiles in one dimension, tj across the posts: a grid in y ends at 65,536 x 64 batch rows.
 __global__ __launch_bounds__(kBlock) void k_transpose_g(const float* __restrict__ g, int32_t batch,
-                                                        int32_t n_post, int32_t Bp,
-                                                        float* __restrict__ gT,
+                                                        int32_t n_post, int32_t Bp, int32_t tj,
+                                                        int32_t tiles, float* __restrict__ gT,
                                                         uint32_t* __restrict__ odd) {
+  constexpr int kS = kBlock / 64;
   __shared__ float s_t[kTr][kTr + 1];
   __shared__ uint32_t s_odd;
   const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
-  const int64_t j0 = (int64_t)blockIdx.x * kTr, b0 = (int64_t)blockIdx.y * kTr;
   if (threadIdx.x == 0) s_odd = 0u;
   __syncthreads();
   bool bad = false;
+  for (int32_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+    const int64_t j0 = (int64_t)(t % tj) * kTr, b0 = (int64_t)(t / tj) * kTr;
 #pragma unroll
-  for (int r = r0; r < kTr; r += kBlock / 64) {
-    const int64_t b = b0 + r, j = j0 + c;
-    const float v = b < batch && j < n_post ? g[b * n_post + j] : 0.0f;
-    bad |= (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u;
-    s_t[r][c] = v;
+    for (int u = 0; u < kTr / kS; ++u) {
+      const int r = r0 + u * kS;
+      const int64_t b = b0 + r, j = j0 + c;
+      const float v = b < batch && j < n_post ? g[b * n_post + j] : 0.0f;
+      bad |= (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u;
+      s_t[r][c] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kTr / kS; ++u) {
+      const int r = r0 + u * kS;
+      const int64_t j = j0 + r, b = b0 + c;
+      if (j <= n_post && b < Bp) gT[j * Bp + b] = s_t[c][r];
+    }
+    __syncthreads();                     // the tile is rewritten next
   }
   if (bad) s_odd = 1u;
   __syncthreads();
-#pragma unroll
-  for (int r = r0; r < kTr; r += kBlock / 64) {
-    const int64_t j = j0 + r, b = b0 + c;
-    if (j <= n_post && b < Bp) gT[j * Bp + b] = s_t[c][r];
-  }
-  if (threadIdx.x == 0) odd[blockIdx.y * gridDim.x + blockIdx.x] = s_odd;  // inf or NaN in it
+  if (threadIdx.x == 0) odd[blockIdx.x] = s_odd;   // an inf or NaN among its values
 }
 
 // One wave per pre row i.
@@ -876,9 +885,8 @@ template <typename T, bool kCsr, bool kHet, int LB>
 __global__ __launch_bounds__(kBlock) void k_matvec_vjp_bt(
     const T* __restrict__ spk, int32_t batch, int32_t n_pre, const int32_t* __restrict__ indptr,
     const int32_t* __restrict__ indices, int32_t k, const float* __restrict__ w, float w_homo,
-    int32_t n_post, const float* __restrict__ g, const float* __restrict__ gT, int32_t Bp,
-    const uint32_t* __restrict__ odd, int32_t n_odd, float* __restrict__ gx,
-    float* __restrict__ gw) {
+    int32_t n_post, const float* __restrict__ gT, int32_t Bp, const uint32_t* __restrict__ odd,
+    int32_t n_odd, float* __restrict__ gx, float* __restrict__ gw) {
   constexpr int G = BS_WAVE / LB, A = LB, kU = 16;
   const int lane = bs_lane();
   const int q = lane / LB, bl = lane % LB;
@@ -998,7 +1006,20 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp_bt(
   }
 }
 
-int32_t vjp_lanes(int32_t batch) { return batch <= 16 ? 16 : 64; }
+// The transposed form of `batch` rows of n_post values: batch columns of gT (whole groups of
+// `lanes`), tiles of the transposition and how many lie across the posts.
+struct VjpBt {
+  int32_t lanes, Bp;
+  int64_t tj, tiles;
+  int32_t wgs() const { return (int32_t)(tiles < kTrWgs ? tiles : kTrWgs); }
+};
+
+VjpBt vjp_bt(int32_t batch, int32_t n_post) {
+  const int32_t lanes = batch <= 16 ? 16 : 64;
+  const int64_t Bp = ((int64_t)batch + lanes - 1) / lanes * lanes;
+  const int64_t tj = ((int64_t)n_post + kTr) / kTr;    // posts and the zero row
+  return VjpBt{lanes, (int32_t)Bp, tj, tj * ((Bp + kTr - 1) / kTr)};
+}
 
 // Workspace of the transposed form, 0 where the per-row form is kept: its extra launch costs
 // ~4 us, which a few batch rows of a small layer do not repay (us per call, per-row /
@@ -1007,11 +1028,11 @@ int32_t vjp_lanes(int32_t batch) { return batch <= 16 ? 16 : 64; }
 size_t vjp_bt_bytes(int32_t batch, int32_t n_pre, int32_t n_post) {
   if (n_pre < 1 || n_post < 1 || batch < 3 || (batch < 8 && (int64_t)batch * n_pre < 20000))
     return 0;
-  const int64_t Bp = ((int64_t)batch + vjp_lanes(batch) - 1) / vjp_lanes(batch) * vjp_lanes(batch);
-  const int64_t n = ((int64_t)n_post + 1) * Bp;
+  if (batch > (1 << 29)) return 0;
+  const VjpBt t = vjp_bt(batch, n_post);
+  const int64_t n = ((int64_t)n_post + 1) * t.Bp;
   if (n >= (1LL << 30)) return 0;                      // 32-bit element offsets
-  const int64_t tiles = ((int64_t)n_post + kTr) / kTr * ((Bp + kTr - 1) / kTr);
-  return (size_t)(n + tiles) * 4;
+  return (size_t)(n + t.wgs()) * 4;
 }
 
 int grid_for(int64_t work_items_waves) {
@@ -1320,18 +1341,17 @@ int vjp_batch(const void* spk, int32_t spk_dtype, int32_t batch, int32_t n_pre,
   if (need > 0 && ws != nullptr) {
     BS_CHECK_ARG(ws_bytes >= need, "bs_event_matvec_vjp_batch_ws_f32: workspace of %zu bytes "
                  "needed (got %zu)", need, ws_bytes);
-    const int32_t lanes = vjp_lanes(batch);
-    const int32_t Bp = (batch + lanes - 1) / lanes * lanes;
+    const VjpBt t = vjp_bt(batch, n_post);
     float* gT = (float*)ws;
-    uint32_t* odd = (uint32_t*)(gT + ((int64_t)n_post + 1) * Bp);
-    const dim3 tg((unsigned)(((int64_t)n_post + kTr) / kTr), (unsigned)((Bp + kTr - 1) / kTr));
-    k_transpose_g<<<tg, kBlock, 0, s>>>(grad_out, batch, n_post, Bp, gT, odd);
+    uint32_t* odd = (uint32_t*)(gT + ((int64_t)n_post + 1) * t.Bp);
+    k_transpose_g<<<t.wgs(), kBlock, 0, s>>>(grad_out, batch, n_post, t.Bp, (int32_t)t.tj,
+                                             (int32_t)t.tiles, gT, odd);
     BS_CHECK_LAUNCH();
 #define BS_BT1(T, C, H, L)                                                                   \
   k_matvec_vjp_bt<T, C, H, L><<<g, kBlock, 0, s>>>((const T*)spk, batch, n_pre, indptr, indices, \
-                                                   k, w, w_homo, n_post, grad_out, gT, Bp, odd, \
-                                                   (int32_t)(tg.x * tg.y), grad_spk, grad_w)
-#define BS_BT(T, C, H) do { if (lanes == 16) BS_BT1(T, C, H, 16); else BS_BT1(T, C, H, 64); } while (0)
+                                                   k, w, w_homo, n_post, gT, t.Bp, odd,       \
+                                                   t.wgs(), grad_spk, grad_w)
+#define BS_BT(T, C, H) do { if (t.lanes == 16) BS_BT1(T, C, H, 16); else BS_BT1(T, C, H, 64); } while (0)
     if (spk_dtype == BS_SPK_U8) {
       if (csr) { if (het) BS_BT(uint8_t, true, true); else BS_BT(uint8_t, true, false); }
       else { if (het) BS_BT(uint8_t, false, true); else BS_BT(uint8_t, false, false); }

@@ -53,3 +53,33 @@ def test_transposed_vjp_equals_rows(B, n_pre, n_post, k, het, csr, odd):
         assert abs(float(gw) - float(total)) <= 1e-5 * absum
     only = ops.event_matvec_vjp_batch(x, idx, w, n_post, g, indptr=indptr, need_w=False)[0]
     assert same(only, gs)
+
+
+def test_more_batch_rows_than_a_grid_has_in_y():
+    """65,537 tiles of 64 batch rows, one past a grid's y limit here: gradients of the few rows that carry any equal the per-row
+    calls, the others are zero."""
+    import torch
+    if not torch.cuda.is_available():
+        pytest.fail('GPU tests need a ROCm GPU')
+    from brainstate_amd import ops
+    B, n_pre, n_post, k = 65_536 * 64 + 1, 2, 3, 5
+    print('[case] vjp batch rows', B, flush=True)
+    rs = np.random.RandomState(4)
+    t = lambda a: torch.as_tensor(np.asarray(a), device='cuda')  # noqa: E731
+    idx = t(rs.randint(0, n_post, (n_pre, k)).astype(np.int32))
+    w = t(rs.randn(n_pre, k).astype(np.float32))
+    x = torch.zeros(B, n_pre, device='cuda')
+    g = torch.zeros(B, n_post, device='cuda')
+    at = [0, 63, 64, 70_000, B // 2, B - 2, B - 1]
+    for b in at:
+        x[b] = t(rs.rand(n_pre).astype(np.float32) + 0.5)
+        g[b] = t(rs.randn(n_post).astype(np.float32))
+    gs, gw = ops.event_matvec_vjp_batch(x, idx, w, n_post, g)
+    total = None
+    for b in at:
+        a, c = ops.event_matvec_vjp(x[b], idx, w, n_post, g[b].contiguous())
+        assert torch.equal(gs[b], a), b
+        total = c if total is None else total + c
+    assert torch.equal(gw, total)
+    gs[at] = 0
+    assert int(torch.count_nonzero(gs)) == 0
