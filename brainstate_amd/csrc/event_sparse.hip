@@ -472,9 +472,11 @@ __global__ __launch_bounds__(kBlock) void k_mv_reduce(int32_t n_post, int32_t R,
 }
 
 // gw[0] += the sum over the workgroup's waves of their (wave-uniform) v: one atomic per
-// workgroup.  The terms of this one sum mostly cancel, so it is carried in 64 bits up to the
-// atomic.  Called by every wave that has not ended.  (One per active row made the shared
-// weight's gradient of 100k rows of 128 synapses take 1.27 ms.)
+// workgroup.  The terms of this one sum mostly cancel, so it is carried in 64 bits over the rows
+// of a workgroup (a row's own sum of g is formed as the kernel forms grad_x, and the workgroups'
+// sums meet in fp32).  Called by every wave that has not ended.  (One fp32 atomic per active
+// row made the shared weight's gradient of 100k rows of 128 synapses take 1.27 ms, and that of
+// two batch rows of 100k x 100 take 266 us; 91 this way.)
 template <int kWaves>
 __device__ __forceinline__ void block_atomic_sum(double v, float* gw) {
   __shared__ double s_v[kWaves];
@@ -774,7 +776,7 @@ __global__ __launch_bounds__(kLvB) void k_matvec_vjp_lds(
 //   grad_x[b, i] as k_matvec_vjp forms it for row b (lane partials, then a wave sum);
 //   grad_w[i, k] = sum_b x[b, i] * g[b, idx[i, k]], the products added in b order, as adding
 //   the per-row gradients one after another does (fp32, no contraction);
-//   homogeneous: grad_w[0] += x[b, i] * sum_k g[b, idx[i, k]] per (row, b), one atomic each.
+//   homogeneous: grad_w[0] += x[b, i] * sum_k g[b, idx[i, k]], summed over (row, b) in 64 bits.
 template <typename T, bool kCsr, bool kHet>
 __global__ __launch_bounds__(kBlock) void k_matvec_vjp_batch(
     const T* __restrict__ spk, int32_t batch, int32_t n_pre, const int32_t* __restrict__ indptr,
@@ -784,6 +786,7 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp_batch(
   const int lane = bs_lane();
   const int64_t nw = (int64_t)gridDim.x * (kBlock / BS_WAVE);
   const int32_t nnz = kCsr ? indptr[n_pre] : 0;
+  double sw = 0.0;
   for (int64_t row = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / BS_WAVE; row < n_pre;
        row += nw) {
     int64_t beg, end;
@@ -811,10 +814,8 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp_batch(
         sx += __shfl_xor(sx, o);
         sg += __shfl_xor(sg, o);
       }
-      if (lane == 0) {
-        if (gx) gx[(int64_t)b * n_pre + row] = sx;
-        if (!kHet && gw && xv != 0.0f) bs_atomic_add_f32(gw, xv * sg);
-      }
+      if (lane == 0 && gx) gx[(int64_t)b * n_pre + row] = sx;
+      if (!kHet && xv != 0.0f) sw += (double)xv * (double)sg;
     }
     if (kHet && gw) {
       for (int64_t s = beg + lane; s < end; s += BS_WAVE) {
@@ -829,6 +830,7 @@ __global__ __launch_bounds__(kBlock) void k_matvec_vjp_batch(
       }
     }
   }
+  if (!kHet && gw) block_atomic_sum<kBlock / BS_WAVE>(sw, gw);
 }
 
 // ---- the same with g transposed: gT[j][b], Bp columns (a multiple of LB), row n_post zero ----
