@@ -11,6 +11,7 @@
 // the spike of each and adds the weight in column order, so every post accumulates its
 // incoming synapses in ascending (pre, k) order -- bit-identical to a sequential pre-major
 // scatter, with no atomics.
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -1023,18 +1024,37 @@ VjpBt vjp_bt(int32_t batch, int32_t n_post) {
   return VjpBt{lanes, (int32_t)Bp, tj, tj * ((Bp + kTr - 1) / kTr)};
 }
 
-// Workspace of the transposed form, 0 where the per-row form is kept: its extra launch costs
-// ~4 us, which a few batch rows of a small layer do not repay (us per call, per-row /
-// transposed: 2 x 3200 rows of 80 12.6 / 14.6, 3 x 500 of 500 13.2 / 17.4, 4 x 3200 of 80
-// 12.3 / 15.4, 8 x 10k of 100 55 / 19, 100 x 500 of 20 87 / 15, 128 x 10k of 100 1020 / 115).
+// Workspace the transposed form takes, 0 where it is never taken (vjp_bt_pays decides for a call).
 size_t vjp_bt_bytes(int32_t batch, int32_t n_pre, int32_t n_post) {
-  if (n_pre < 1 || n_post < 1 || batch < 3 || (batch < 8 && (int64_t)batch * n_pre < 20000))
-    return 0;
-  if (batch > (1 << 29)) return 0;
+  if (n_pre < 1 || n_post < 1 || batch < 3 || batch > (1 << 29)) return 0;
   const VjpBt t = vjp_bt(batch, n_post);
   const int64_t n = ((int64_t)n_post + 1) * t.Bp;
   if (n >= (1LL << 30)) return 0;                      // 32-bit element offsets
   return (size_t)(n + t.wgs()) * 4;
+}
+
+// Whether the transposed form is the faster one, for rows of k synapses (their mean for CSR;
+// unknown, k < 1: 64), from the costs of both in us.  Per-row kernel: a wave walks its rows'
+// chunks of 64 synapses once per batch row, one after another, or the gathers of g are the
+// limit (slower once g outgrows the L2).  Transposed: the transposition at 2 (16 lanes) or 4
+// TB/s, then a chunk per lane group.  Measured (us per call, per-row / transposed, K
+// synapses a row): 3 x (7000 -> 10k, K = 20) 6.3 / 11.2, the same -> 1M 12.5 / 48.9; 8 x (500 ->
+// 400k, K = 20) 7.8 / 30.6; 17 x (500 -> 100k, K = 20) 15.0 / 21.4, 64 rows of it 70 / 25; 8 x
+// (10k -> 500, K = 20) 15.2 / 12.3; 16 x (5000 -> 1M, K = 100) 205 / 69; 64 x (3200 -> 4000, K =
+// 80) 95 / 23; 64 x (500 -> 10k, K = 1000) 509 / 72.
+bool vjp_bt_pays(int32_t batch, int32_t n_pre, int32_t n_post, int32_t k) {
+  const VjpBt t = vjp_bt(batch, n_post);
+  const double kk = k > 0 ? k : 64, waves = 64.0 * bs_num_cus();
+  const double rounds = std::ceil(n_pre / waves), chunks = std::ceil(kk / BS_WAVE);
+  const double visit = (double)batch * n_post * 4 > 32e6 ? 2.4e-5 : 6e-6;
+  const double row = 2.0 + std::fmax(rounds * batch * (0.45 + 0.4 * chunks),
+                                     (double)batch * n_pre * kk * visit);
+  const bool narrow = t.lanes == 16;
+  const double move = ((double)batch + t.Bp) * n_post * 4 / (narrow ? 2e6 : 4e6);
+  const double bt = 8.0 + move +
+                    std::fmax(rounds * (t.Bp / t.lanes) * chunks * (narrow ? 1.7 : 3.4),
+                              (double)t.Bp * n_pre * kk * 0.8e-6);
+  return bt < row;
 }
 
 int grid_for(int64_t work_items_waves) {
@@ -1340,7 +1360,7 @@ int vjp_batch(const void* spk, int32_t spk_dtype, int32_t batch, int32_t n_pre,
   }
   const int g = grid_for(n_pre);
   const size_t need = vjp_bt_bytes(batch, n_pre, n_post);
-  if (need > 0 && ws != nullptr) {
+  if (need > 0 && ws != nullptr && vjp_bt_pays(batch, n_pre, n_post, k)) {
     BS_CHECK_ARG(ws_bytes >= need, "bs_event_matvec_vjp_batch_ws_f32: workspace of %zu bytes "
                  "needed (got %zu)", need, ws_bytes);
     const VjpBt t = vjp_bt(batch, n_post);

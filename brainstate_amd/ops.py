@@ -219,6 +219,8 @@ def event_matvec_vjp_batch(spk, indices, w, n_post, grad_out, k=None, indptr=Non
     if need_w:
         gw = torch.empty((), dtype=torch.float32, device=dev) if homo else \
             torch.empty(w.shape, dtype=torch.float32, device=dev)
+    if indptr is not None:   # the mean row length: which form is the faster one depends on it
+        k = -(-indices.numel() // max(n_pre, 1))
     nbytes = int(N.lib().bs_event_matvec_vjp_batch_workspace_size(B, n_pre, int(n_post)))
     ws = _call_workspace(nbytes, dev)
     N.check(N.lib().bs_event_matvec_vjp_batch_ws_f32(

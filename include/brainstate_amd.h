@@ -149,8 +149,9 @@ BS_API int bs_matvec_ws_f32(const void* spk, int32_t spk_dtype, int32_t value, i
                             void* workspace, size_t workspace_bytes, bs_stream_t stream);
 
 /* The same gradients with a workspace of bs_event_matvec_vjp_batch_workspace_size bytes, in
- * which grad_out is held transposed (0: none is used).  grad_spk and per-synapse grad_w have
- * the bits bs_event_matvec_vjp_batch_f32 gives. */
+ * which grad_out is held transposed when that is the faster form (0: never).  grad_spk and
+ * per-synapse grad_w have the bits bs_event_matvec_vjp_batch_f32 gives.  With indptr, k is a
+ * hint for that choice: the mean row length, or 0. */
 BS_API size_t bs_event_matvec_vjp_batch_workspace_size(int32_t batch, int32_t n_pre,
                                                        int32_t n_post);
 BS_API int bs_event_matvec_vjp_batch_ws_f32(const void* spk, int32_t spk_dtype, int32_t batch,
