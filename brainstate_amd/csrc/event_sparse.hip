@@ -279,10 +279,12 @@ __global__ __launch_bounds__(kBlock) void k_matvec(const T* __restrict__ spk, in
 // The mat-vec (fixed fan-out) with the sums in LDS instead of global fp32 atomics, which run at
 // ~2e10/s over the whole chip.  Workgroup (range q, row group r) of batch row blockIdx.y lists
 // its active rows, reads all their synapses and adds those that hit its `len` posts; with one
-// row group it writes the outputs, else a partial row that k_mv_reduce adds (header, then
+// row group it writes the outputs, else a partial row that k_mv_finish adds (header, then
 // [R][n_post] per batch row).  As in the bucketed operator, the row groups in use follow the
 // spikes: every workgroup estimates the active synapses from the same leading rows, groups
-// past R_eff return, and R_eff = 1 writes the outputs.
+// past R_eff return, and R_eff = 1 writes the outputs.  When the estimate says that atomics are
+// the faster way for so few events (MvCost), the workgroups clear the outputs instead, R_eff is
+// 0 and k_mv_finish adds the events.
 // A shared event weight is counted and added in one chain afterwards (the sequential sum, as
 // k_matvec and the bucketed operator give it); other sums are fp32 in no fixed order.
 // The workgroups of a row group read the same synapses: they are placed on one XCD.
@@ -291,15 +293,60 @@ __global__ __launch_bounds__(kBlock) void k_matvec(const T* __restrict__ spk, in
 constexpr int kMvB = 1024;
 constexpr int kMvPosts = 16000;        // posts per range at most (two workgroups per CU)
 constexpr int kMvSpan = 4096;          // rows listed at a time
-constexpr int kMvSample = 16384;       // leading rows the estimate reads
+constexpr int kMvSample = 4096;        // spikes the estimate reads: one load per thread
 constexpr int kMvSyn = 8192;           // active synapses per row group the estimate aims for,
                                        // plus n_post / 4 (a group's partials cost that much)
 constexpr int kMvHdr = 64;             // header words ahead of a batch row's partials
+
+// Costs in us of the two ways, from the events ev of a batch row (filled in by mv_plan).
+struct MvCost {
+  int32_t R, rs;       // row groups at most, and with one span of rows each
+  float per;           // events of a batch row per spike of the sample
+  float group;         // 1 / events a row group aims for
+  float direct0, direct1, lds0, span, last, read, part;
+  // row groups for ev events: no group lists more than one span of rows if R allows
+  __host__ __device__ int32_t groups(float ev) const {
+    const int32_t re = (int32_t)fminf(ceilf(ev * group), (float)R);
+    const int32_t g = re > rs ? re : rs;
+    return g > R ? R : g;
+  }
+  // atomics: a rate; LDS: spans of rows listed one after another, then the synapses of a
+  // group's events, then its partial sums
+  __host__ __device__ float direct_us(float ev) const { return direct0 + ev * direct1; }
+  __host__ __device__ float lds_us(float ev, int32_t g) const {
+    return lds0 + (g >= rs ? span : last) + read * (ev / (float)g) +
+           (g > 1 ? (float)g * part : 0.0f);
+  }
+};
+
+// Batch rows the estimate reads with `sample` threads, kE spikes each, on one of them.
+__host__ __device__ __forceinline__ int32_t mv_sample_rows(int32_t sample, int32_t kE) {
+  const int32_t n = kMvSample / kE / sample;
+  return n < 1 ? 1 : n;
+}
+
+struct __attribute__((packed, aligned(1))) Any16 {
+  uint4 v;
+};
+
+// Nonzero ones among 16 bytes of spikes.
+template <typename T>
+__device__ __forceinline__ int32_t nonzeros(uint4 v) {
+  const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+  int32_t c = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (sizeof(T) == 4) c += (x[e] & 0x7fffffffu) != 0u;
+    else c += __popc((((x[e] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x[e]) & 0x80808080u);
+  }
+  return c;
+}
 template <typename T, bool kHet, bool kVal>
 __global__ __launch_bounds__(kMvB) void k_mv_lds(
     const T* __restrict__ spk, int32_t n_pre, const int32_t* __restrict__ indices, int32_t k,
     const float* __restrict__ w, float w_homo, int32_t n_post, int32_t nr, int32_t len,
-    int32_t R, int32_t accumulate, float* __restrict__ out, uint32_t* __restrict__ ws) {
+    int32_t R, int32_t sample, MvCost cost, int32_t accumulate, float* __restrict__ out,
+    uint32_t* __restrict__ ws) {
   constexpr bool kCount = !kHet && !kVal;
   constexpr int kWv = kMvB / BS_WAVE, kU = kMvSpan / kMvB;
   __shared__ __align__(16) uint32_t s_acc[kMvPosts];
@@ -307,6 +354,7 @@ __global__ __launch_bounds__(kMvB) void k_mv_lds(
   __shared__ int32_t s_wave[kU][kWv];
   const int lane = bs_lane();
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / BS_WAVE));
+  const T* all = spk;
   spk += (int64_t)blockIdx.y * n_pre;
   out += (int64_t)blockIdx.y * n_post;
   ws += (int64_t)blockIdx.y * (kMvHdr + (R > 1 ? (int64_t)R * n_post : 0));
@@ -314,14 +362,18 @@ __global__ __launch_bounds__(kMvB) void k_mv_lds(
   const int32_t x = blockIdx.x;
   const int32_t r = R == 1 ? 0 : x / (8 * nr) * 8 + x % 8, q = R == 1 ? x : x / 8 % nr;
   if (r >= R) return;
+  const int32_t p0 = q * len;
+  const int32_t rest = n_post - p0 > 0 ? n_post - p0 : 0;     // 0: a last range left empty
+  const int32_t pn = rest < len ? rest : len;
   int32_t Reff = 1;
-  if (R > 1) {
-    const int32_t ns = n_pre < kMvSample ? n_pre : kMvSample;
+  if (sample > 0) {                    // threads per batch row, 16 bytes of its spikes each
+    constexpr int32_t kE = 16 / sizeof(T);
+    const int32_t b = (int32_t)threadIdx.x / sample, i = (int32_t)threadIdx.x % sample * kE;
     int32_t c = 0;
-#pragma unroll
-    for (int u = 0; u < kMvSample / kMvB; ++u) {
-      const int32_t i = u * kMvB + threadIdx.x;
-      c += i < ns && spk[i < ns ? i : 0] != T(0) ? 1 : 0;
+    if (b < (int32_t)gridDim.y && b < mv_sample_rows(sample, kE)) {
+      const T* p = all + (int64_t)b * n_pre;
+      if (i + kE <= n_pre) c = nonzeros<T>(((const Any16*)(p + i))->v);
+      else for (int32_t e = i; e < n_pre; ++e) c += p[e] != T(0) ? 1 : 0;
     }
 #pragma unroll
     for (int o = BS_WAVE / 2; o > 0; o >>= 1) c += __shfl_xor(c, o);
@@ -331,27 +383,38 @@ __global__ __launch_bounds__(kMvB) void k_mv_lds(
 #pragma unroll
     for (int v = 0; v < kWv; ++v) c += s_wave[0][v];
     __syncthreads();
-    const double syn = (double)c * (double)n_pre / (double)ns * (double)k;
-    // ... and no group lists more than one span of rows
-    const double re = ceil(syn / (kMvSyn + n_post / 4)), rs = ceil((double)n_pre / kMvSpan);
-    const double rw = re > rs ? re : rs;
-    Reff = rw > (double)R ? R : (int32_t)rw;
+    const float ev = (float)c * cost.per;               // the same in every workgroup, so all
+                                                        // batch rows take the same way
+    Reff = cost.groups(ev);
+    if (cost.direct_us(ev) < cost.lds_us(ev, Reff)) Reff = 0;
     if (x == 0 && threadIdx.x == 0) ws[0] = (uint32_t)Reff;
+    if (Reff == 0) {                   // this workgroup's share of its range cleared
+      if (accumulate) return;
+      const int32_t j0 = (int32_t)((int64_t)pn * r / R), j1 = (int32_t)((int64_t)pn * (r + 1) / R);
+      for (int32_t j = j0 + threadIdx.x; j < j1; j += kMvB) out[p0 + j] = 0.0f;
+      return;
+    }
     if (r >= Reff) return;             // whole workgroup
   }
-  const int32_t p0 = q * len;
-  const int32_t rest = n_post - p0 > 0 ? n_post - p0 : 0;     // 0: a last range left empty
-  const int32_t pn = rest < len ? rest : len;
   for (int j = threadIdx.x; j < pn; j += kMvB) s_acc[j] = 0u;
   const int64_t r0 = (int64_t)n_pre * r / Reff, r1 = (int64_t)n_pre * (r + 1) / Reff;
+  T next[kU];                          // the next span's spikes, in flight over this one's rows
+  auto ahead = [&](int64_t c0) {
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int64_t i = c0 + u * kMvB + threadIdx.x;
+      next[u] = spk[i < r1 ? i : r0];  // repeated past the end
+    }
+  };
+  if (r0 < r1) ahead(r0);
   for (int64_t c0 = r0; c0 < r1; c0 += kMvSpan) {
     uint64_t m[kU];
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
-      const int64_t i = c0 + u * kMvB + threadIdx.x;
-      m[u] = bs_ballot(i < r1 && spk[i < r1 ? i : r0] != T(0));
+      m[u] = bs_ballot(c0 + u * kMvB + threadIdx.x < r1 && next[u] != T(0));
       if (lane == 0) s_wave[u][wid] = __popcll(m[u]);
     }
+    if (c0 + kMvSpan < r1) ahead(c0 + kMvSpan);
     __syncthreads();                   // also: s_acc is zero, the last span's rows are done
     int32_t count = 0;
 #pragma unroll
@@ -427,22 +490,72 @@ __global__ __launch_bounds__(kMvB) void k_mv_lds(
   }
 }
 
-// out[j] = (accumulate ? out[j] : 0) + the R_eff partials of j.  A workgroup takes 64 posts;
-// thread (c, j) adds every fourth partial from c on, 16 in flight, and the four sums meet in
-// order.
-template <bool kCount>
-__global__ __launch_bounds__(kBlock) void k_mv_reduce(int32_t n_post, int32_t R, float w_homo,
-                                                      int32_t accumulate,
-                                                      const uint32_t* __restrict__ ws,
-                                                      float* __restrict__ out) {
-  constexpr int kC = kBlock / BS_WAVE, kF = 16;
+// R_eff > 1: out[j] = (accumulate ? out[j] : 0) + the R_eff partials of j.  A workgroup takes 64
+// posts; thread (c, j) adds every fourth partial from c on, 16 in flight, and the four sums meet
+// in order.  R_eff = 0: a workgroup lists the active ones of its `rows` pre rows and adds their
+// synapses to the outputs with global atomics, a wave 4 x 64 of one row at a time (k_matvec
+// gives a wave the whole row: 12.1 us for 12 rows of 1,000 synapses, 10.0 here for both launches).
+template <typename T, bool kHet, bool kVal>
+__global__ __launch_bounds__(kBlock) void k_mv_finish(
+    const T* __restrict__ spk, int32_t n_pre, int32_t rows, const int32_t* __restrict__ indices,
+    int32_t k, const float* __restrict__ w, int32_t n_post, int32_t R, float w_homo,
+    int32_t accumulate, const uint32_t* __restrict__ ws, float* __restrict__ out) {
+  constexpr bool kCount = !kHet && !kVal;
+  constexpr int kC = kBlock / BS_WAVE, kF = 16, kQ = 4;
   __shared__ uint32_t s_p[kC][BS_WAVE];
-  const int c = threadIdx.x / BS_WAVE, lane = bs_lane();
-  const int64_t j = (int64_t)blockIdx.x * BS_WAVE + lane;
-  ws += (int64_t)blockIdx.y * (kMvHdr + (int64_t)R * n_post);
+  __shared__ int32_t s_rows[kRowsCap];
+  const int c = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / BS_WAVE)), lane = bs_lane();
+  ws += (int64_t)blockIdx.y * (kMvHdr + (R > 1 ? (int64_t)R * n_post : 0));
   out += (int64_t)blockIdx.y * n_post;
   const int32_t Reff = (int32_t)__builtin_amdgcn_readfirstlane(ws[0]);
-  if (Reff <= 1) return;
+  if (Reff == 0) {
+    spk += (int64_t)blockIdx.y * n_pre;
+    const int64_t r0 = (int64_t)blockIdx.x * rows;
+    int32_t count = 0;
+    for (int32_t off = 0; off < rows; off += kBlock) {
+      const int64_t r = r0 + off + threadIdx.x;
+      const bool a = off + (int32_t)threadIdx.x < rows && r < n_pre && spk[r] != T(0);
+      const uint64_t m = bs_ballot(a);
+      if (lane == 0) s_p[c][0] = (uint32_t)__popcll(m);
+      __syncthreads();
+      int32_t pos = count;
+#pragma unroll
+      for (int v = 0; v < kC; ++v) {
+        const int32_t n = (int32_t)s_p[v][0];
+        pos += v < c ? n : 0;
+        count += n;
+      }
+      if (a) s_rows[pos + bs_rank_below(m)] = (int32_t)r;
+      __syncthreads();
+    }
+    const int32_t per = (k - 1) / (kQ * BS_WAVE) + 1;        // items of a row
+    for (int32_t a = 0, q = c;; q += kC) {                   // item q of active row a
+      while (q >= per && a < count) {
+        q -= per;
+        ++a;
+      }
+      if (a >= count) break;
+      const int32_t row = __builtin_amdgcn_readfirstlane(s_rows[a]);
+      const float xv = kVal ? (float)spk[row] : 1.0f;
+      const int32_t t0 = q * (kQ * BS_WAVE) + lane;
+      int32_t jj[kQ];
+      float vv[kQ];
+#pragma unroll
+      for (int u = 0; u < kQ; ++u) {
+        const int32_t t = t0 + u * BS_WAVE;
+        const int64_t o = (int64_t)row * k + t;
+        jj[u] = t < k ? indices[o] : -1;
+        vv[u] = kHet && t < k ? w[o] : w_homo;
+      }
+#pragma unroll
+      for (int u = 0; u < kQ; ++u)
+        if ((uint32_t)jj[u] < (uint32_t)n_post)
+          bs_atomic_add_f32(out + jj[u], kVal ? vv[u] * xv : vv[u]);
+    }
+    return;
+  }
+  const int64_t j = (int64_t)blockIdx.x * BS_WAVE + lane;
+  if (Reff == 1 || (int64_t)blockIdx.x * BS_WAVE >= n_post) return;
   const uint32_t* p = ws + kMvHdr + (j < n_post ? j : 0);
   float sum = 0.0f;
   uint32_t cnt = 0;
@@ -1167,25 +1280,35 @@ extern "C" int bs_event_gather_f32(const uint32_t* spk_bits, int32_t n_pre,
 
 namespace {
 
-// Ranges and row groups of k_mv_lds; R = 0 where k_matvec is kept.  k_matvec costs ~12 us (with
-// the fill of its outputs) plus 5e-5 us per event, k_mv_lds ~20 us on a sparse layer and
-// 1e-5 us per event (us per call, k_matvec / k_mv_lds): 100k x 100k, K = 1000, p = 0.1 529 /
-// 125, 0.01 65 / 34, 0.002 19 / 23; one shared weight, 400k x 4k, K = 250, p = 0.2 870 / 119,
-// 0.002 23 / 19; 64 x 3200 -> 4000, K = 80, p = 0.05 43 / 17, 0.002 11 / 9; 128 x 10k, K = 100,
-// p = 0.2 1207 / 179.  The density is not known here: single vectors take it from 2e7
-// synapses (5e7 with a shared weight, whose calls are otherwise the shortest), batches of 8
-// (32) always; more than 8 ranges would read the synapses too often.
+// Ranges and row groups of k_mv_lds; R = 0 where k_matvec is kept: below 2e7 synapses (5e7 events
+// of a shared weight; 2e6 for batches of 8, or 32), where its two launches cost more than the
+// atomics they save, past 8 ranges, and where the costs say that LDS would not win with a
+// quarter of the rows active.  Elsewhere the estimate decides on the device.  A batch with one
+// row group each and few spans takes no estimate: its single launch is the shorter way from
+// p ~ 0.01 on, and must promise twice the atomics' speed.
+// us per call, k_matvec / LDS always / as decided here, at p = 0.002, 0.01, 0.05:
+//   100k x 100k, K = 1000          19.7/23/20   69/28/26    272/83/76
+//   250k x 100k, K = 100            7.9/34/14   19/37/24     70/43/36
+//   250k x 4000, K = 100            9.5/16/12   28/19/17    116/27/25
+//   8 x (20k -> 20k, K = 100)       6.9/23/11   14/27/17     46/29/27
+//   64 x (3200 -> 4000, K = 80)     6.8/9.7/9.4 13/13/13     43/18/17
+//   128 x (200k -> 20k, K = 100)   249/322/240  1209/573/471 6035/1150/1026
+//   16 x (2000 -> 128k, K = 20)     6.0/43/5.9  6.2/47/6.2   8.0/51/8.0
+// The constants below are fits to such calls.
 struct MvPlan {
   int32_t nr, len, R;
+  int32_t sample;                      // threads per batch row of the estimate; 0: LDS always
+  MvCost cost;
 };
 
-MvPlan mv_plan(int32_t batch, int32_t n_pre, int32_t k, int32_t n_post, bool csr, bool count) {
-  MvPlan p{0, 0, 0};
-  if (csr || batch < 1 || n_pre < 1 || n_post < 1 || k < 1) return p;
+MvPlan mv_plan(int32_t batch, int32_t n_pre, int32_t k, int32_t n_post, bool csr, bool count,
+               int32_t kE) {
+  MvPlan p{};
+  if (csr || batch < 1 || n_pre < 1 || n_post < 1 || k < 1 || k >= (1 << 30)) return p;
   const int32_t least = (n_post + kMvPosts - 1) / kMvPosts;
   if (least > 8) return p;
-  const double syn = (double)n_pre * k;
-  if (batch < (count ? 32 : 8) && syn * batch < (count ? 5e7 : 2e7)) return p;
+  const double syn = (double)n_pre * k * batch;
+  if (syn < (batch >= (count ? 32 : 8) ? 2e6 : (count ? 5e7 : 2e7))) return p;
   int32_t nr = least, R = 1;
   if (batch >= 8) {
     const int32_t want = 512 / batch < 8 ? 512 / batch : 8;
@@ -1200,11 +1323,45 @@ MvPlan mv_plan(int32_t batch, int32_t n_pre, int32_t k, int32_t n_post, bool csr
     R = (int32_t)(g < rows ? g : rows);
     if (R < 1) R = 1;
   }
-  return MvPlan{nr, (n_post + nr - 1) / nr, R};
+  const int32_t spans = ((n_pre - 1) / R) / kMvSpan + 1;         // of each of R groups
+  const double rounds = R > 1 ? 1.0 : std::ceil((double)wgs / 512);
+  MvCost& c = p.cost;
+  c.R = R;
+  c.rs = (n_pre - 1) / kMvSpan + 1;
+  const int32_t threads = kMvSample / kE, need = (n_pre - 1) / kE + 1;
+  p.sample = threads / batch < 1 ? 1 : threads / batch;
+  p.sample = p.sample < need ? p.sample : need;
+  const int32_t rows = mv_sample_rows(p.sample, kE) < batch ? mv_sample_rows(p.sample, kE) : batch;
+  const int64_t seen = (int64_t)p.sample * kE < n_pre ? (int64_t)p.sample * kE : n_pre;
+  c.per = (float)((double)n_pre / (double)(seen * rows) * k);
+  c.group = 1.0f / (float)(kMvSyn + n_post / 4);
+  c.direct0 = 9.0f;
+  c.direct1 = (float)(batch * 5.4e-5 + 0.16 / n_post);
+  c.lds0 = batch > 1 ? 11.0f : 4.0f;
+  c.span = (float)(5.5 * rounds);
+  c.last = c.span * (float)spans;
+  c.read = (float)(rounds * ((count ? 0.3e-3 : 1.4e-3) / nr +
+                             (0.03 + 0.003 * ((k - 1) / BS_WAVE + 1)) / k));
+  c.part = (float)((double)batch * n_post * 2.4e-6);
+  if (R == 1 && rounds * spans < 9) p.sample = 0;
+  const float dense = 0.25f * (float)n_pre * (float)k, most = c.lds_us(dense, c.groups(dense));
+  if (c.direct_us(dense) < (p.sample ? 1.3f : 2.0f) * most) return MvPlan{};
+  p.nr = nr;
+  p.len = (n_post + nr - 1) / nr;
+  p.R = R;
+  return p;
 }
 
 size_t mv_ws_bytes(const MvPlan& p, int32_t batch, int32_t n_post) {
-  return p.R > 1 ? (size_t)batch * (kMvHdr + (size_t)p.R * n_post) * 4 : 0;
+  return p.sample ? (size_t)batch * (kMvHdr + (p.R > 1 ? (size_t)p.R * n_post : 0)) * 4 : 0;
+}
+
+// Pre rows per workgroup of k_matvec and of k_mv_finish's atomics: enough workgroups (over all
+// batch rows) to fill the chip, at most kRowsCap rows each.
+int32_t matvec_rows(int32_t batch, int32_t n_pre) {
+  const int64_t g = (int64_t)bs_num_cus() * 4;
+  const int64_t rows = ((int64_t)n_pre * batch + g - 1) / g;
+  return (int32_t)(rows < 64 ? 64 : (rows > kRowsCap ? kRowsCap : rows));
 }
 
 // Shared launcher of the fused mat-vec (event or value-weighted).
@@ -1219,29 +1376,34 @@ int matvec_launch(const void* spk, int32_t spk_dtype, int32_t batch, int32_t n_p
   BS_CHECK_ARG(spk_dtype == BS_SPK_U8 || spk_dtype == BS_SPK_F32, "%s: unknown spike dtype %d",
                who, spk_dtype);
   if (n_post > 0) BS_CHECK_ARG(out != nullptr, "%s: out is NULL", who);
-  const MvPlan mp = mv_plan(batch, n_pre, k, n_post, indptr != nullptr, !kVal && w == nullptr);
+  const MvPlan mp = mv_plan(batch, n_pre, k, n_post, indptr != nullptr, !kVal && w == nullptr,
+                            spk_dtype == BS_SPK_U8 ? 16 : 4);
   const size_t mneed = mv_ws_bytes(mp, batch, n_post);
   if (mp.R > 0 && (mneed == 0 || ws != nullptr)) {
     BS_CHECK_ARG(spk && indices, "%s: NULL pointer", who);
     BS_CHECK_ARG(ws_bytes >= mneed, "%s: workspace of %zu bytes needed (got %zu)", who, mneed,
                  ws_bytes);
     const dim3 mg((unsigned)(mp.R == 1 ? mp.nr : (mp.R + 7) / 8 * 8 * mp.nr), (unsigned)batch);
-    const dim3 rg((unsigned)(((int64_t)n_post + BS_WAVE - 1) / BS_WAVE), (unsigned)batch);
     uint32_t* part = (uint32_t*)ws;
+    const int32_t rows = matvec_rows(batch, n_pre);
+    const int64_t gp = mp.R > 1 ? ((int64_t)n_post + BS_WAVE - 1) / BS_WAVE : 1;
+    const int64_t gr = ((int64_t)n_pre + rows - 1) / rows;
+    const dim3 fg((unsigned)(gp > gr ? gp : gr), (unsigned)batch);
 #define BS_ML(T, H)                                                                        \
-  k_mv_lds<T, H, kVal><<<mg, kMvB, 0, s>>>((const T*)spk, n_pre, indices, k, w, w_homo, n_post, \
-                                           mp.nr, mp.len, mp.R, accumulate, out, part)
+  do {                                                                                     \
+    k_mv_lds<T, H, kVal><<<mg, kMvB, 0, s>>>((const T*)spk, n_pre, indices, k, w, w_homo,    \
+                                             n_post, mp.nr, mp.len, mp.R, mp.sample, mp.cost, \
+                                             accumulate, out, part);                       \
+    BS_CHECK_LAUNCH();                                                                     \
+    if (mp.sample)                                                                         \
+      k_mv_finish<T, H, kVal><<<fg, kBlock, 0, s>>>((const T*)spk, n_pre, rows, indices, k, w, \
+                                                    n_post, mp.R, w_homo, accumulate, part,  \
+                                                    out);                                  \
+  } while (0)
     if (spk_dtype == BS_SPK_U8) { if (w) BS_ML(uint8_t, true); else BS_ML(uint8_t, false); }
     else { if (w) BS_ML(float, true); else BS_ML(float, false); }
 #undef BS_ML
     BS_CHECK_LAUNCH();
-    if (mp.R > 1) {
-      if (w || kVal)
-        k_mv_reduce<false><<<rg, kBlock, 0, s>>>(n_post, mp.R, w_homo, accumulate, part, out);
-      else
-        k_mv_reduce<true><<<rg, kBlock, 0, s>>>(n_post, mp.R, w_homo, accumulate, part, out);
-      BS_CHECK_LAUNCH();
-    }
     return BS_OK;
   }
   if (!accumulate) {
@@ -1250,18 +1412,13 @@ int matvec_launch(const void* spk, int32_t spk_dtype, int32_t batch, int32_t n_p
   }
   if (n_pre == 0 || n_post == 0 || (indptr == nullptr && k == 0)) return BS_OK;
   BS_CHECK_ARG(spk && indices, "%s: NULL pointer", who);
-  // rows per workgroup: enough workgroups (over all batch rows) to fill the chip, at most
-  // kRowsCap rows each
-  int64_t g = (int64_t)bs_num_cus() * 4;
-  int64_t rows = ((int64_t)n_pre * batch + g - 1) / g;
-  if (rows < 64) rows = 64;
-  if (rows > kRowsCap) rows = kRowsCap;
-  g = ((int64_t)n_pre + rows - 1) / rows;
+  const int32_t rows = matvec_rows(batch, n_pre);
+  const int64_t g = ((int64_t)n_pre + rows - 1) / rows;
   const size_t shm = n_post <= kLdsPosts ? (size_t)n_post * sizeof(float) : 0;
   const bool het = w != nullptr, csr = indptr != nullptr;
 #define BS_MV(T, C, H)                                                                \
   k_matvec<T, C, H, kVal><<<dim3((unsigned)g, (unsigned)batch), kBlock, shm, s>>>(       \
-      (const T*)spk, n_pre, (int32_t)rows, indptr, indices, k, w, w_homo, n_post, out)
+      (const T*)spk, n_pre, rows, indptr, indices, k, w, w_homo, n_post, out)
   if (spk_dtype == BS_SPK_U8) {
     if (csr) { if (het) BS_MV(uint8_t, true, true); else BS_MV(uint8_t, true, false); }
     else { if (het) BS_MV(uint8_t, false, true); else BS_MV(uint8_t, false, false); }
@@ -1318,7 +1475,7 @@ extern "C" int bs_value_matvec_batch_f32(const float* x, int32_t batch, int32_t 
 extern "C" size_t bs_matvec_workspace_size(int32_t batch, int32_t n_pre, int32_t k,
                                            int32_t n_post, int32_t count) {
   bs_clear_error();
-  return mv_ws_bytes(mv_plan(batch, n_pre, k, n_post, false, count != 0), batch, n_post);
+  return mv_ws_bytes(mv_plan(batch, n_pre, k, n_post, false, count != 0, 4), batch, n_post);
 }
 
 extern "C" int bs_matvec_ws_f32(const void* spk, int32_t spk_dtype, int32_t value, int32_t batch,
