@@ -751,7 +751,7 @@ __global__ __launch_bounds__(kSB) void k_bucket_scatter(
   if (count > 0) flush(!listed);
   __syncthreads();  // s_acc complete (and zeroed, for a group without active rows)
   if (kSingle && blockIdx.x == 0 && threadIdx.x == 0) {  // the hint, from the exact count
-    *hdr = 1;
+    if (hdr && blockIdx.y == 0) *hdr = 1;
     const uint32_t e = (n_act + kActivePer - 1) / kActivePer;
     if (est_out) *est_out = e < 1u ? 1 : (e > (uint32_t)Rmax ? Rmax : (int32_t)e);
   }
@@ -1199,7 +1199,7 @@ extern "C" size_t bs_event_bucket_batch_workspace_size(int32_t batch, int32_t n_
   bs_clear_error();
   if (batch <= 0 || n_pre <= 0 || n_post <= 0 || nb <= 0) return 0;
   const int32_t R = batch_row_groups(batch, n_pre, nb);
-  return (size_t)batch * (kHdr + (R > 1 ? (size_t)R * n_post * sizeof(uint32_t) : 0));
+  return R > 1 ? (size_t)batch * (kHdr + (size_t)R * n_post * sizeof(uint32_t)) : 0;
 }
 
 extern "C" int bs_event_bucket_batch_f32(const void* spk, int32_t spk_dtype, int32_t batch,
@@ -1224,13 +1224,14 @@ extern "C" int bs_event_bucket_batch_f32(const void* spk, int32_t spk_dtype, int
                "%s: f32 spikes not 4-byte aligned", fn);
   BS_CHECK_ARG(lw == nullptr || qexp != nullptr, "%s: qexp is NULL", fn);
   const int32_t R = batch_row_groups(batch, n_pre, nb);
-  const size_t need = (size_t)batch * (kHdr + (R > 1 ? (size_t)R * n_post * sizeof(uint32_t) : 0));
-  BS_CHECK_ARG(workspace != nullptr && workspace_bytes >= need,
+  const size_t need = bs_event_bucket_batch_workspace_size(batch, n_pre, n_post, nb);
+  BS_CHECK_ARG(need == 0 || (workspace != nullptr && workspace_bytes >= need),
                "%s: workspace of %zu bytes needed (got %zu)", fn, need,
                workspace ? workspace_bytes : (size_t)0);
   BS_CHECK_ARG((uintptr_t)workspace % 8 == 0, "%s: workspace not 8-byte aligned", fn);
-  int32_t* hdr = (int32_t*)workspace;  // one header per batch row, then the partials
-  uint32_t* part = (uint32_t*)((char*)workspace + (size_t)batch * kHdr);
+  // one header per batch row, then the partials; the single launch (R = 1) takes neither
+  int32_t* hdr = R > 1 ? (int32_t*)workspace : nullptr;
+  uint32_t* part = R > 1 ? (uint32_t*)((char*)workspace + (size_t)batch * kHdr) : nullptr;
   int32_t nsub = 1;
   if (R == 1) {
     const int64_t per = kTargetWgs / ((int64_t)nb * batch);

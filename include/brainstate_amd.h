@@ -215,7 +215,7 @@ BS_API int bs_event_bucket_f32(const void* spk, int32_t spk_dtype, int32_t n_pre
 
 /* bs_event_bucket_f32 for `batch` spike rows spk [batch, n_pre] onto out [batch, n_post] in one
  * or two launches: every row gets the bits bs_event_bucket_f32 gives it (any mode).  At most
- * 65535 rows; the workspace needs bs_event_bucket_batch_workspace_size bytes. */
+ * 65535 rows; the workspace needs bs_event_bucket_batch_workspace_size bytes (0: none). */
 BS_API size_t bs_event_bucket_batch_workspace_size(int32_t batch, int32_t n_pre, int32_t n_post,
                                                    int32_t nb);
 BS_API int bs_event_bucket_batch_f32(const void* spk, int32_t spk_dtype, int32_t batch,
