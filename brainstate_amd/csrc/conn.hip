@@ -17,7 +17,7 @@
 // counting the accepted draws on the way (a word budget of expected draws + 12 standard
 // deviations); k_mt_place ranks and places every accepted draw.  8e7 draws below 1e6 (135k
 // blocks): one workgroup twisting every block, then passes to temper, count, scan and place,
-// took 42.5 ms; this form 0.51 ms (jumps 117 us, twists 190, placing 147 = 4.5 TB/s).
+// took 42.5 ms; this form 0.49 ms (263 segments: jumps 115 us, twists 192, placing 154 = 4.2 TB/s).
 //
 // Without replacement (allow_multi_conn=False) the reference uses its JAX generator
 // (init_indices_without_replace, :39-62), which cannot be reproduced without JAX.  Here each
@@ -480,17 +480,19 @@ int jump_parts(int64_t srcs) {
 
 // Segments of 2^m blocks.  Few long segments leave the chip idle while they twist, many
 // short ones cost a jump each, and every level of jumps is a launch that regenerates 33 blocks:
-// m minimises the three, with their measured costs (15 us per level, 38 us per target and
-// workgroup, 0.33 / 0.56 / 0.9 us per block with 1 / 2 / 4 segments on a compute unit).  For
-// 135k blocks m = 8 / 9 / 10 took 470 / 455 / 560 us of kernels; short streams stay in one
-// segment (below ~70 blocks) or few (430 blocks, 256k draws: 205 us in one, 91 in 14).
+// m minimises the sum, with costs fitted to kernel traces (a level 12.5 us and (34 + 25 per
+// target of a source) / parts; twisting 0.32 / 0.385 / 0.485 / 0.61 us per block with 1 .. 4
+// segments on a compute unit).  For 134k blocks m = 8 / 9 / 10 take 193 + 124 / 115 + 192 /
+// 91 + 327 us of jumps + twists (508 / 491 / 597 us per call); short streams stay in one
+// segment (below ~70 blocks) or few (430 blocks, 256k draws: 165 us in one, 80 in 14).
 struct MtPlan {
   int m, levels;
   int32_t segs;
 };
 
 MtPlan mt_plan(int64_t blocks) {
-  constexpr double kLevelUs = 15.0, kJumpUs = 38.0;
+  constexpr double kLevelUs = 12.5, kSourceUs = 34.0, kTargetUs = 25.0;
+  constexpr double kTwistUs[] = {0.32, 0.385, 0.485, 0.61};
   constexpr int64_t kMaxSegs = 1024, kCus = 256;
   MtPlan best{0, 0, 0};
   double cost = 0.0;
@@ -498,12 +500,12 @@ MtPlan mt_plan(int64_t blocks) {
     const int64_t segs = (blocks + (1LL << m) - 1) >> m;
     if (segs > kMaxSegs) continue;
     int levels = 0;
-    double c = (double)(segs > 1 ? 1LL << m : blocks) *
-               (0.12 + 0.2 * (double)((segs + kCus - 1) / kCus));
+    double c = (double)(segs > 1 ? 1LL << m : blocks) * kTwistUs[(segs - 1) / kCus];
     for (int64_t nsrc = 1; nsrc < segs; nsrc *= 4, ++levels) {
       const int64_t srcs = segs - nsrc < nsrc ? segs - nsrc : nsrc;
       const int64_t tgts = (segs < 4 * nsrc ? segs : 4 * nsrc) - nsrc;
-      c += kLevelUs + kJumpUs / jump_parts(srcs) * (double)((tgts + srcs - 1) / srcs);
+      c += kLevelUs + (kSourceUs + kTargetUs * (double)((tgts + srcs - 1) / srcs)) /
+                          jump_parts(srcs);
     }
     if (best.segs == 0 || c < cost) {
       best = MtPlan{m, levels, (int32_t)segs};

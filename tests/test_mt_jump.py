@@ -57,3 +57,19 @@ def test_jump_polynomials_reproduce_the_stream(tmp_path):
     assert out.returncode == 0, out
     state = np.random.RandomState(5489).get_state()[1]
     assert out.stdout.split() == [str(state[1]), str(state[623]), '0']
+
+
+# draws, bound and the segments their stream is cut into: the plans measured as the fastest
+@pytest.mark.parametrize('n_pre,k,n_post,segs', [(800_000, 100, 1_000_000, 263),
+                                                 (200_000, 80, 200_000, 263),
+                                                 (3200, 80, 4000, 14), (100, 100, 4000, 1)])
+def test_segments_of_a_stream(n_pre, k, n_post, segs):
+    import math
+
+    from brainstate_amd import _native as N
+    p = n_post / 2.0 ** (n_post - 1).bit_length()
+    words = int(n_pre * k / p + 12 * math.sqrt(n_pre * k * (1 - p)) / p) + 2 * 624
+    blocks = -(-words // 624)
+    pad = lambda n: -(-n // 256) * 256  # noqa: E731
+    size = lambda s: pad(blocks * 2496) + pad(blocks * 4) + pad(s * 4) + pad(s * 2496) + 256  # noqa: E731
+    assert N.lib().bs_conn_fixed_num_workspace_size(n_pre, k, n_post, 0) == size(segs)
