@@ -74,8 +74,10 @@ def _record(fn, *args):
     """Apply the autograd Function ``fn``.  torch binds the arguments of a Function with its own
     ``setup_context`` to the forward's signature on every call (~30 us); outside torch.func
     transforms, which need that form, the same Function with the context passed to
-    ``forward`` is applied instead (same saved tensors, ``backward`` and ``jvp``)."""
-    if torch._C._are_functorch_transforms_active():
+    ``forward`` is applied instead (same saved tensors, ``backward`` and ``jvp``).  A torch
+    that cannot tell whether a transform is active gets the form that always holds."""
+    active = getattr(torch._C, '_are_functorch_transforms_active', None)
+    if active is None or active():
         return fn.apply(*args)
     return fn._direct.apply(*args)
 
