@@ -1280,6 +1280,14 @@ extern "C" int bs_event_gather_f32(const uint32_t* spk_bits, int32_t n_pre,
 
 namespace {
 
+// Pre rows per workgroup of k_matvec and of k_mv_finish's atomics: enough workgroups (over all
+// batch rows) to fill the chip, at most kRowsCap rows each.
+int32_t matvec_rows(int32_t batch, int32_t n_pre) {
+  const int64_t g = (int64_t)bs_num_cus() * 4;
+  const int64_t rows = ((int64_t)n_pre * batch + g - 1) / g;
+  return (int32_t)(rows < 64 ? 64 : (rows > kRowsCap ? kRowsCap : rows));
+}
+
 // Ranges and row groups of k_mv_lds; R = 0 where k_matvec is kept: below 2e7 synapses (5e7 events
 // of a shared weight; 2e6 for batches of 8, or 32), where its two launches cost more than the
 // atomics they save, past 8 ranges, and where the costs say that LDS would not win with a
@@ -1336,7 +1344,11 @@ MvPlan mv_plan(int32_t batch, int32_t n_pre, int32_t k, int32_t n_post, bool csr
   c.per = (float)((double)n_pre / (double)(seen * rows) * k);
   c.group = 1.0f / (float)(kMvSyn + n_post / 4);
   c.direct0 = 9.0f;
-  c.direct1 = (float)(batch * 5.4e-5 + 0.16 / n_post);
+  // few pre rows leave few workgroups for the atomics, 5e-3 us an event each (4000 rows of
+  // 10,000 synapses at p = 0.1 take 487 us in k_matvec, 70 here; 200 of 200,000 17 ms, 1.4 ms)
+  const int32_t per_wg = matvec_rows(batch, n_pre);
+  c.direct1 = (float)std::fmax(batch * 5.4e-5 + 0.16 / n_post,
+                               5e-3 / ((n_pre - 1) / per_wg + 1));
   c.lds0 = batch > 1 ? 11.0f : 4.0f;
   c.span = (float)(5.5 * rounds);
   c.last = c.span * (float)spans;
@@ -1354,14 +1366,6 @@ MvPlan mv_plan(int32_t batch, int32_t n_pre, int32_t k, int32_t n_post, bool csr
 
 size_t mv_ws_bytes(const MvPlan& p, int32_t batch, int32_t n_post) {
   return p.sample ? (size_t)batch * (kMvHdr + (p.R > 1 ? (size_t)p.R * n_post : 0)) * 4 : 0;
-}
-
-// Pre rows per workgroup of k_matvec and of k_mv_finish's atomics: enough workgroups (over all
-// batch rows) to fill the chip, at most kRowsCap rows each.
-int32_t matvec_rows(int32_t batch, int32_t n_pre) {
-  const int64_t g = (int64_t)bs_num_cus() * 4;
-  const int64_t rows = ((int64_t)n_pre * batch + g - 1) / g;
-  return (int32_t)(rows < 64 ? 64 : (rows > kRowsCap ? kRowsCap : rows));
 }
 
 // Shared launcher of the fused mat-vec (event or value-weighted).

@@ -65,3 +65,25 @@ def test_way_follows_density(B, n_pre, n_post, k, kind, p, sdt):
         bound = (n + 2) * 2.0 ** -24 * (size + base[b].double().abs()) + 1e-30
         assert bool(((outs[0][b].double() - want).abs() <= bound).all()), b
         assert bool(((outs[1][b].double() - want - base[b].double()).abs() <= bound).all()), b
+
+
+def test_few_long_rows_take_lds():
+    """60 rows of 50,000 synapses in 8 batch rows: one workgroup per batch row could add them by
+    atomics (1,007 us at p = 0.1), so the outputs are summed in LDS (109), with the same sums."""
+    import torch
+    if not torch.cuda.is_available():
+        pytest.fail('GPU tests need a ROCm GPU')
+    from brainstate_amd import ops
+    print('[case] mv long rows', flush=True)
+    gen = torch.Generator(device='cuda').manual_seed(2)
+    B, n_pre, n_post, k = 8, 60, 5000, 50_000
+    idx = torch.randint(0, n_post, (n_pre, k), device='cuda', generator=gen, dtype=torch.int32)
+    x = (torch.rand(B, n_pre, device='cuda', generator=gen) < 0.2).float()
+    # integer weights: every sum is exact
+    w = torch.randint(-3, 4, (n_pre, k), device='cuda', generator=gen).float()
+    out = ops.value_matvec(x, idx, w, n_post)
+    for b in range(B):
+        want = torch.zeros(n_post, device='cuda')
+        for r in x[b].nonzero().reshape(-1):
+            want.index_add_(0, idx[r].long(), w[r])
+        assert torch.equal(out[b], want), b

@@ -7,12 +7,13 @@ pytestmark = pytest.mark.gpu
 
 
 # single vectors: one range, the most ranges, a last range cut to nothing, many rows per group,
-# one row group; batches: a few row groups each, one, and posts in slices of a few outputs
+# one row group; batches: a few row groups each, one, and posts in slices of a few outputs (small
+# ones stay with k_matvec)
 @pytest.mark.parametrize('B,n_pre,n_post,k,p', [
     (0, 400_000, 17, 125, 0.01), (0, 50_001, 128_000, 1001, 0.03), (0, 50_000, 16_001, 1000, 0.002),
     (0, 100_003, 3, 500, 0.0), (0, 60, 90_000, 900_000, 0.5), (8, 4097, 16_000, 33, 0.3),
     (33, 1000, 300, 64, 0.5), (64, 3200, 4000, 80, 0.05), (9, 8200, 20_003, 65, 1.0),
-    (130, 5, 1, 3, 0.6)])
+    (130, 5, 1, 3, 0.6), (260, 2000, 5, 40, 0.3)])
 @pytest.mark.parametrize('kind', ['event', 'value', 'event_shared', 'value_shared'])
 @pytest.mark.parametrize('sdt', ['u8', 'f32'])
 def test_matvec_lds(B, n_pre, n_post, k, p, kind, sdt):
