@@ -6,13 +6,33 @@ C entry point of include/brainstate_amd.h and raises ``NativeError`` on failure.
 import ctypes
 import functools
 import math
+import threading
 
 import numpy as np
 import torch
 
 from . import _native as N
 
+# Workspaces kept per (device, stream).  Those of compactions and of the bucketed operator stay
+# when a call outgrows them (each is at least twice the last, so together they are less than
+# the largest): a captured graph may use them.  The lock is held from the choice of a workspace
+# to the end of the native call, which runs without the GIL, so that the two launches of one
+# thread's call have none of another's on the same stream between them.
 _WS_CACHE = {}
+_WS_OUTGROWN = []
+_WS_LOCK = threading.Lock()
+
+
+def _kept_workspace(key, nbytes, device, alloc):
+    """The workspace kept under ``key``, of at least ``nbytes``; ``alloc`` (torch.empty or
+    torch.zeros) makes a new one.  Called with _WS_LOCK held."""
+    ws = _WS_CACHE.get(key)
+    if ws is None or ws.numel() < nbytes:
+        if ws is not None:
+            _WS_OUTGROWN.append(ws)
+            nbytes = max(nbytes, 2 * ws.numel())
+        ws = _WS_CACHE[key] = alloc(nbytes, dtype=torch.uint8, device=device)
+    return ws
 
 
 def _spk_dtype(spk):
@@ -33,12 +53,9 @@ def _spk_view(spk):
 def compact_workspace(n, device):
     """Zero-filled workspace for bs_spike_compact, cached per (device, stream, size)."""
     nbytes = int(N.lib().bs_spike_compact_workspace_size(int(n)))
-    key = (device.index, N.raw_stream(device))
-    ws = _WS_CACHE.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.zeros(max(nbytes, 4096), dtype=torch.uint8, device=device)
-        _WS_CACHE[key] = ws
-    return ws
+    with _WS_LOCK:
+        return _kept_workspace((device.index, N.raw_stream(device)), max(nbytes, 4096), device,
+                               torch.zeros)
 
 
 def spike_compact(spk):
@@ -439,15 +456,12 @@ def event_bucket(spk, layout, out=None, accumulate=False, mode='auto'):
     if out is None:
         out = torch.empty(L['n_post'], dtype=torch.float32, device=dev)
     sh = N.raw_stream(dev)
-    key = ('bucket', dev.index, sh)
-    ws = _WS_CACHE.get(key)
-    if nbytes > 0 and (ws is None or ws.numel() < nbytes):
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-        _WS_CACHE[key] = ws
-    N.check(N.lib().bs_event_bucket_f32(
-        N.ptr(spk), _spk_dtype(spk), *fixed, N.ptr(out), 1 if accumulate else 0,
-        N.ptr(ws) if nbytes > 0 else None, nbytes, m, hint[2], ctypes.c_void_p(sh)),
-        'bs_event_bucket_f32')
+    with _WS_LOCK:
+        ws = _kept_workspace(('bucket', dev.index, sh), nbytes, dev, torch.empty) \
+            if nbytes > 0 else None
+        N.check(N.lib().bs_event_bucket_f32(
+            N.ptr(spk), _spk_dtype(spk), *fixed, N.ptr(out), 1 if accumulate else 0,
+            N.ptr(ws), nbytes, m, hint[2], ctypes.c_void_p(sh)), 'bs_event_bucket_f32')
     return out
 
 

@@ -68,3 +68,61 @@ def test_calls_on_one_stream_have_workspaces_of_their_own(monkeypatch, call, gro
     (a, na), (b, nb) = lib.seen
     assert a + na <= b or b + nb <= a, 'two calls in flight share a workspace'
     assert not ops._WS_CACHE                  # nothing that a later, larger call could replace
+
+
+class _Kept:
+    """bs_event_bucket_f32 replaced: notes the workspaces, and a call that starts while another
+    is inside."""
+
+    def __init__(self):
+        self.seen, self.inside, self.overlap = [], 0, False
+        self.entered, self.go = threading.Event(), threading.Event()
+
+    def bs_event_bucket_f32(self, *a):
+        self.overlap |= self.inside > 0
+        self.inside += 1
+        self.seen.append((a[-5].value, a[-4]))
+        if len(self.seen) == 1:
+            self.entered.set()
+            self.go.wait(20)
+        self.inside -= 1
+        return 0
+
+    def bs_spike_compact_workspace_size(self, n):
+        return 8 * n
+
+
+def test_kept_workspaces_stay_and_calls_do_not_interleave(monkeypatch):
+    lib = _Kept()
+    monkeypatch.setattr(N, 'lib', lambda: lib)
+    monkeypatch.setattr(N, 'raw_stream', lambda device=None: 7)
+    monkeypatch.setattr(ops, '_WS_CACHE', {})
+    monkeypatch.setattr(ops, '_WS_OUTGROWN', [], raising=False)
+    monkeypatch.setattr(ops, '_bucket_hint', lambda L: (None, [1], None))
+    monkeypatch.setattr(ops, 'bucket_auto_mode', lambda L: 'split')
+    t = torch.zeros(3, 2, dtype=torch.int32)
+
+    def call(nbytes):
+        L = dict(seg=t, lidx=t, w=None, qexp=None, n_pre=3, n_post=4)
+        L['_call'] = ((), nbytes, (t, t, None, None), 1)
+        ops.event_bucket(torch.ones(3, dtype=torch.uint8), L)
+
+    first = threading.Thread(target=call, args=(4096,))
+    second = threading.Thread(target=call, args=(4096,))
+    first.start()
+    assert lib.entered.wait(20)
+    second.start()
+    second.join(0.2)
+    lib.go.set()
+    first.join(20)
+    second.join(20)
+    assert not lib.overlap and len(lib.seen) == 2
+    call(5000)                                # outgrows the first: both stay allocated
+    call(100_000)
+    kept = [lib.seen[0], lib.seen[2], lib.seen[3]]
+    alive = {w.data_ptr(): w.numel() for w in [*ops._WS_OUTGROWN, *ops._WS_CACHE.values()]}
+    assert all(alive.get(p, 0) >= n for p, n in kept) and len({p for p, _ in kept}) == 3
+    sizes = sorted(alive.values())
+    assert all(b >= 2 * a for a, b in zip(sizes, sizes[1:]))
+    small, large = (ops.compact_workspace(n, torch.device('cpu')) for n in (10, 10_000))
+    assert small is ops._WS_OUTGROWN[-1] and large.numel() >= 80_000
