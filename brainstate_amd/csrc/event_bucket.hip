@@ -278,8 +278,9 @@ __global__ void k_bucket_qexp(const uint32_t* wmax, const uint32_t* dmax, int32_
 // 16 bytes of spikes (16 u8 rows or 4 f32 rows) of block blk = rows [blk*E, blk*E + E), rows
 // outside [r0, r1) read as 0: one vector load when the whole block lies inside (of any
 // alignment: a batch row of an odd length starts anywhere), else one load per row in range.
-// The per-row form, out of line: it runs only for a block cut by the range, and kept inline its code (in every load slot) would be fetched by the instruction
-// cache on every path (measured: 5x the misses of a compact kernel, ~2 us of a dense step).
+// The per-row form, out of line: it runs only for a block cut by the range, and kept inline its
+// code (in every load slot) would be fetched by the instruction cache on every path (measured:
+// 5x the misses of a compact kernel, ~2 us of a dense step).
 template <typename T>
 __device__ __noinline__ uint4 spike_block_rows(const T* __restrict__ spk, uint32_t row,
                                                uint32_t r0, uint32_t r1) {

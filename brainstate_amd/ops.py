@@ -117,7 +117,7 @@ def _fixed_matvec(x, value, indices, k, w, n_post, out, accumulate, batch, n_pre
         nb = min(65535, batch - b0)
         nbytes = int(lib.bs_matvec_workspace_size(nb, n_pre, k, n_post,
                                                   1 if homo and not value else 0))
-        ws = _call_workspace(nbytes, dev)
+        ws = _call_workspace(nbytes, dev) if nbytes else None
         xs, ys = (x, out) if nb == batch else (x.reshape(batch, n_pre)[b0:b0 + nb],
                                                out.reshape(batch, n_post)[b0:b0 + nb])
         N.check(lib.bs_matvec_ws_f32(
@@ -484,7 +484,7 @@ def event_bucket_batch(spk, layout, out=None, accumulate=False):
         nb = min(65535, B - b0)
         nbytes = int(N.lib().bs_event_bucket_batch_workspace_size(nb, n_pre, L['n_post'],
                                                                   L['nb']))
-        ws = _call_workspace(nbytes, dev)
+        ws = _call_workspace(nbytes, dev) if nbytes else None
         N.check(N.lib().bs_event_bucket_batch_f32(
             N.ptr(spk[b0:b0 + nb]), _spk_dtype(spk), nb, *fixed, N.ptr(out[b0:b0 + nb]),
             1 if accumulate else 0, N.ptr(ws), nbytes, ctypes.c_void_p(sh)),
