@@ -17,7 +17,7 @@
 // counting the accepted draws on the way (a word budget of expected draws + 12 standard
 // deviations); k_mt_place ranks and places every accepted draw.  8e7 draws below 1e6 (135k
 // blocks): one workgroup twisting every block, then passes to temper, count, scan and place,
-// took 42.5 ms; this form 0.49 ms (263 segments: jumps 115 us, twists 192, placing 154 = 4.2 TB/s).
+// took 42.5 ms; this form 0.50 ms (263 segments: jumps 115 us, twists 189, placing 145 = 4.5 TB/s).
 //
 // Without replacement (allow_multi_conn=False) the reference uses its JAX generator
 // (init_indices_without_replace, :39-62), which cannot be reproduced without JAX.  Here each
