@@ -1140,6 +1140,7 @@ VjpBt vjp_bt(int32_t batch, int32_t n_post) {
 // Workspace the transposed form takes, 0 where it is never taken (vjp_bt_pays decides for a call).
 size_t vjp_bt_bytes(int32_t batch, int32_t n_pre, int32_t n_post) {
   if (n_pre < 1 || n_post < 1 || batch < 3 || batch > (1 << 29)) return 0;
+  if (batch < 8 && (int64_t)batch * n_pre < 20000) return 0;   // rarely pays: not worth the memory
   const VjpBt t = vjp_bt(batch, n_post);
   const int64_t n = ((int64_t)n_post + 1) * t.Bp;
   if (n >= (1LL << 30)) return 0;                      // 32-bit element offsets
