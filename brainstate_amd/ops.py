@@ -13,11 +13,11 @@ import torch
 
 from . import _native as N
 
-# Workspaces kept per (device, stream).  Those of compactions and of the bucketed operator stay
-# when a call outgrows them (each is at least twice the last, so together they are less than
-# the largest): a captured graph may use them.  The lock is held from the choice of a workspace
-# to the end of the native call, which runs without the GIL, so that the two launches of one
-# thread's call have none of another's on the same stream between them.
+# Workspaces kept per (device, stream).  One that a call outgrows stays as well (each is at least
+# twice the last, so together they are less than the largest): a captured graph may use it.  The
+# lock guards the choice; for the bucketed operator it is held to the end of the native call,
+# which runs without the GIL, so that the two launches of one thread's call have none of
+# another's on the same stream between them (the others are one launch).
 _WS_CACHE = {}
 _WS_OUTGROWN = []
 _WS_LOCK = threading.Lock()
@@ -510,21 +510,16 @@ def event_dense(spk, W, float_as_event=True, out=None):
     nbytes, tick = _dense_ws(B, n_in, n_out)
     ws = None
     if nbytes > 0:
-        # ticket counters lead the workspace: zero on entry, left zero by every call; the
-        # bytes after them hold partial sums, so bytes past the previous call's counters
-        # are zeroed before a call that needs more counters
-        key = ('dense', W.device.index, N.raw_stream(W.device))
-        ws, zero = _WS_CACHE.get(key, (None, 0))
-        if ws is None or ws.numel() < nbytes:
-            ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=W.device)
-            zero = ws.numel()
-        if tick > zero:
-            ws[zero:tick].zero_()
-        _WS_CACHE[key] = (ws, tick)
+        # ticket counters lead the workspace: zero on entry, left zero by every call; the bytes
+        # after them hold partial sums.  One workspace per size of the counters (a multiple of
+        # 256 bytes; few of them, since a sum is only split while tiles are few), so no call's
+        # partial sums fall on counters that another one, or a captured one, expects to be zero
+        with _WS_LOCK:
+            ws = _kept_workspace(('dense', W.device.index, N.raw_stream(W.device), tick), nbytes,
+                                 W.device, torch.zeros)
     N.check(N.lib().bs_event_dense_f32(N.ptr(s2), _spk_dtype(s2), B, n_in, N.ptr(W.contiguous()),
-                                       n_out, 1 if float_as_event else 0, N.ptr(out),
-                                       N.ptr(ws) if ws is not None else None, nbytes,
-                                       N.stream_handle(W.device)), 'bs_event_dense_f32')
+                                       n_out, 1 if float_as_event else 0, N.ptr(out), N.ptr(ws),
+                                       nbytes, N.stream_handle(W.device)), 'bs_event_dense_f32')
     return out[0] if squeeze else out
 
 

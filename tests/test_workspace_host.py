@@ -126,3 +126,49 @@ def test_kept_workspaces_stay_and_calls_do_not_interleave(monkeypatch):
     assert all(b >= 2 * a for a, b in zip(sizes, sizes[1:]))
     small, large = (ops.compact_workspace(n, torch.device('cpu')) for n in (10, 10_000))
     assert small is ops._WS_OUTGROWN[-1] and large.numel() >= 80_000
+
+
+def test_dense_counters_are_never_under_partial_sums(monkeypatch):
+    """bs_event_dense_f32 finds its leading ticket counters zero, whatever ran before: a call with
+    fewer counters writes its partial sums into other memory, and outgrown workspaces stay."""
+    class Lib:
+        seen = []
+
+        def bs_event_dense_workspace_size(self, B, n_in, n_out):
+            return self.bs_event_dense_ticket_bytes(B, n_in, n_out) + 4 * B * n_out
+
+        def bs_event_dense_ticket_bytes(self, B, n_in, n_out):
+            return 256 * -(-n_out // 64)
+
+        def bs_event_dense_f32(self, spk, dt, B, n_in, W, n_out, fae, out, ws, nbytes, stream):
+            import ctypes
+            tick = self.bs_event_dense_ticket_bytes(B, n_in, n_out)
+            view = (ctypes.c_uint8 * nbytes).from_address(ws.value)
+            assert not any(view[:tick])
+            for i in range(tick, nbytes):            # partial sums; the counters are left zero
+                view[i] = 1
+            self.seen.append((ws.value, nbytes))
+            return 0
+
+    lib = Lib()
+    monkeypatch.setattr(N, 'lib', lambda: lib)
+    monkeypatch.setattr(N, 'raw_stream', lambda device=None: 7)
+    monkeypatch.setattr(ops, '_WS_CACHE', {})
+    monkeypatch.setattr(ops, '_WS_OUTGROWN', [])
+    ops._dense_ws.cache_clear()
+    try:
+        def call(B, n_out):
+            ops.event_dense(torch.ones(B, 5), torch.ones(5, n_out))
+            return lib.seen[-1]
+
+        captured = call(4, 200)                      # four blocks of counters
+        call(4, 10)                                  # one
+        call(8000, 200)                              # outgrows the first
+        call(4, 300)
+        import ctypes
+        ptr, nbytes = captured                       # its replay, later
+        alive = {w.data_ptr(): w.numel() for w in [*ops._WS_OUTGROWN, *ops._WS_CACHE.values()]}
+        assert alive.get(ptr, 0) >= nbytes
+        assert not any((ctypes.c_uint8 * 1024).from_address(ptr))
+    finally:
+        ops._dense_ws.cache_clear()
