@@ -281,10 +281,10 @@ __global__ __launch_bounds__(kBlock) void k_matvec(const T* __restrict__ spk, in
 // its active rows, reads all their synapses and adds those that hit its `len` posts; with one
 // row group it writes the outputs, else a partial row that k_mv_finish adds (header, then
 // [R][n_post] per batch row).  As in the bucketed operator, the row groups in use follow the
-// spikes: every workgroup estimates the active synapses from the same leading rows, groups
-// past R_eff return, and R_eff = 1 writes the outputs.  When the estimate says that atomics are
-// the faster way for so few events (MvCost), the workgroups clear the outputs instead, R_eff is
-// 0 and k_mv_finish adds the events.
+// spikes: every workgroup estimates the active synapses from the same spikes (the leading ones
+// of every batch row), groups past R_eff return, and R_eff = 1 writes the outputs.  When the
+// estimate says that atomics are the faster way for so few events (MvCost), the workgroups
+// clear the outputs instead, R_eff is 0 and k_mv_finish adds the events.
 // A shared event weight is counted and added in one chain afterwards (the sequential sum, as
 // k_matvec and the bucketed operator give it); other sums are fp32 in no fixed order.
 // The workgroups of a row group read the same synapses: they are placed on one XCD.
@@ -341,6 +341,7 @@ __device__ __forceinline__ int32_t nonzeros(uint4 v) {
   }
   return c;
 }
+
 template <typename T, bool kHet, bool kVal>
 __global__ __launch_bounds__(kMvB) void k_mv_lds(
     const T* __restrict__ spk, int32_t n_pre, const int32_t* __restrict__ indices, int32_t k,

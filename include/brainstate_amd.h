@@ -140,7 +140,8 @@ BS_API int bs_event_matvec_vjp_batch_f32(const void* spk, int32_t spk_dtype, int
 /* bs_event_matvec_batch_f32 (value = 0) or bs_value_matvec_batch_f32 (value = 1) of a fixed
  * fan-out connectivity with a workspace of bs_matvec_workspace_size bytes (0: none is used;
  * count = 1 for events of one shared weight, else 0), in which large layers keep partial sums
- * instead of adding to `out` atomically. */
+ * instead of adding to `out` atomically when the spikes, of which some are counted on the
+ * device, are dense enough for that to be the faster way. */
 BS_API size_t bs_matvec_workspace_size(int32_t batch, int32_t n_pre, int32_t k, int32_t n_post,
                                        int32_t count);
 BS_API int bs_matvec_ws_f32(const void* spk, int32_t spk_dtype, int32_t value, int32_t batch,
