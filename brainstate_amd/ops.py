@@ -97,6 +97,13 @@ def _batch_of(x):
     return lead, math.prod(lead), int(x.shape[-1]) if x.dim() else 1
 
 
+@functools.lru_cache(maxsize=512)
+def _ws_bytes(query, *sizes):
+    """Workspace bytes from the entry point ``query``: a function of the sizes on one kind of
+    device, asked once for each (the call costs 1 us)."""
+    return int(getattr(N.lib(), query)(*sizes))
+
+
 def _call_workspace(nbytes, device):
     """Uninitialised workspace of one call (None for 0 bytes), returned to torch's allocator
     behind the call's kernels.  Not kept per stream: a captured graph would go on using it
@@ -115,8 +122,8 @@ def _fixed_matvec(x, value, indices, k, w, n_post, out, accumulate, batch, n_pre
     lib = N.lib()
     for b0 in range(0, batch, 65535):
         nb = min(65535, batch - b0)
-        nbytes = int(lib.bs_matvec_workspace_size(nb, n_pre, k, n_post,
-                                                  1 if homo and not value else 0))
+        nbytes = _ws_bytes('bs_matvec_workspace_size', nb, n_pre, k, n_post,
+                           1 if homo and not value else 0)
         ws = _call_workspace(nbytes, dev) if nbytes else None
         xs, ys = (x, out) if nb == batch else (x.reshape(batch, n_pre)[b0:b0 + nb],
                                                out.reshape(batch, n_post)[b0:b0 + nb])
@@ -238,7 +245,7 @@ def event_matvec_vjp_batch(spk, indices, w, n_post, grad_out, k=None, indptr=Non
             torch.empty(w.shape, dtype=torch.float32, device=dev)
     if indptr is not None:   # the mean row length: which form is the faster one depends on it
         k = -(-indices.numel() // max(n_pre, 1))
-    nbytes = int(N.lib().bs_event_matvec_vjp_batch_workspace_size(B, n_pre, int(n_post)))
+    nbytes = _ws_bytes('bs_event_matvec_vjp_batch_workspace_size', B, n_pre, int(n_post))
     ws = _call_workspace(nbytes, dev)
     N.check(N.lib().bs_event_matvec_vjp_batch_ws_f32(
         N.ptr(spk), _spk_dtype(spk), B, n_pre, N.ptr(indptr), N.ptr(indices.contiguous()), k,
@@ -482,21 +489,14 @@ def event_bucket_batch(spk, layout, out=None, accumulate=False):
     sh = N.raw_stream(dev)
     for b0 in range(0, B, 65535):
         nb = min(65535, B - b0)
-        nbytes = int(N.lib().bs_event_bucket_batch_workspace_size(nb, n_pre, L['n_post'],
-                                                                  L['nb']))
+        nbytes = _ws_bytes('bs_event_bucket_batch_workspace_size', nb, n_pre, L['n_post'],
+                           L['nb'])
         ws = _call_workspace(nbytes, dev) if nbytes else None
         N.check(N.lib().bs_event_bucket_batch_f32(
             N.ptr(spk[b0:b0 + nb]), _spk_dtype(spk), nb, *fixed, N.ptr(out[b0:b0 + nb]),
             1 if accumulate else 0, N.ptr(ws), nbytes, ctypes.c_void_p(sh)),
             'bs_event_bucket_batch_f32')
     return out
-
-
-@functools.lru_cache(maxsize=256)
-def _dense_ws(B, n_in, n_out):
-    """(workspace bytes, ticket bytes) of bs_event_dense_f32: functions of the shape alone."""
-    return (int(N.lib().bs_event_dense_workspace_size(B, n_in, n_out)),
-            int(N.lib().bs_event_dense_ticket_bytes(B, n_in, n_out)))
 
 
 def event_dense(spk, W, float_as_event=True, out=None):
@@ -507,9 +507,10 @@ def event_dense(spk, W, float_as_event=True, out=None):
     n_out = W.shape[1]
     if out is None:
         out = torch.empty(B, n_out, dtype=torch.float32, device=W.device)
-    nbytes, tick = _dense_ws(B, n_in, n_out)
+    nbytes = _ws_bytes('bs_event_dense_workspace_size', B, n_in, n_out)
     ws = None
     if nbytes > 0:
+        tick = _ws_bytes('bs_event_dense_ticket_bytes', B, n_in, n_out)
         # ticket counters lead the workspace: zero on entry, left zero by every call; the bytes
         # after them hold partial sums.  One workspace per size of the counters (a multiple of
         # 256 bytes; few of them, since a sum is only split while tiles are few), so no call's

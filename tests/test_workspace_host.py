@@ -2,6 +2,7 @@
 between its launches (the library is entered without the GIL), or a larger call after a graph was
 captured, must not be handed, or free, the memory an earlier call's kernels use (CPU, with the
 native library replaced)."""
+import ctypes
 import threading
 
 import pytest
@@ -9,6 +10,13 @@ import torch
 
 from brainstate_amd import _native as N
 from brainstate_amd import ops
+
+
+@pytest.fixture(autouse=True)
+def _sizes_asked_anew():
+    ops._ws_bytes.cache_clear()
+    yield
+    ops._ws_bytes.cache_clear()
 
 
 class _Lib:
@@ -60,6 +68,7 @@ def test_calls_on_one_stream_have_workspaces_of_their_own(monkeypatch, call, gro
     first.start()
     assert lib.entered.wait(20)
     lib.size += grow
+    ops._ws_bytes.cache_clear()
     try:
         run()                                 # while the first call is inside the library
     finally:
@@ -141,7 +150,6 @@ def test_dense_counters_are_never_under_partial_sums(monkeypatch):
             return 256 * -(-n_out // 64)
 
         def bs_event_dense_f32(self, spk, dt, B, n_in, W, n_out, fae, out, ws, nbytes, stream):
-            import ctypes
             tick = self.bs_event_dense_ticket_bytes(B, n_in, n_out)
             view = (ctypes.c_uint8 * nbytes).from_address(ws.value)
             assert not any(view[:tick])
@@ -155,20 +163,15 @@ def test_dense_counters_are_never_under_partial_sums(monkeypatch):
     monkeypatch.setattr(N, 'raw_stream', lambda device=None: 7)
     monkeypatch.setattr(ops, '_WS_CACHE', {})
     monkeypatch.setattr(ops, '_WS_OUTGROWN', [])
-    ops._dense_ws.cache_clear()
-    try:
-        def call(B, n_out):
-            ops.event_dense(torch.ones(B, 5), torch.ones(5, n_out))
-            return lib.seen[-1]
 
-        captured = call(4, 200)                      # four blocks of counters
-        call(4, 10)                                  # one
-        call(8000, 200)                              # outgrows the first
-        call(4, 300)
-        import ctypes
-        ptr, nbytes = captured                       # its replay, later
-        alive = {w.data_ptr(): w.numel() for w in [*ops._WS_OUTGROWN, *ops._WS_CACHE.values()]}
-        assert alive.get(ptr, 0) >= nbytes
-        assert not any((ctypes.c_uint8 * 1024).from_address(ptr))
-    finally:
-        ops._dense_ws.cache_clear()
+    def call(B, n_out):
+        ops.event_dense(torch.ones(B, 5), torch.ones(5, n_out))
+        return lib.seen[-1]
+
+    ptr, nbytes = call(4, 200)                   # four blocks of counters; captured, say
+    call(4, 10)                                  # one
+    call(8000, 200)                              # outgrows the first
+    call(4, 300)
+    alive = {w.data_ptr(): w.numel() for w in [*ops._WS_OUTGROWN, *ops._WS_CACHE.values()]}
+    assert alive.get(ptr, 0) >= nbytes
+    assert not any((ctypes.c_uint8 * 1024).from_address(ptr))
